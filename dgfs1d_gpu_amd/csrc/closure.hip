@@ -902,14 +902,38 @@ k_wgrad_thin(int nb, const float* __restrict__ s1, const __bf16* __restrict__ t3
     }
 }
 
-// out[i] = sum_c part[c][i] (fixed order), i < len
+// out[i] = sum_c part[c][i], i < len, and bout[i] = sum_c bpart[c][i], i < blen
+// (the weight and the bias partials of one layer, nchunk of each), in a fixed
+// order: RO outputs per work-group, each summed by 256 / RO threads over
+// every (256 / RO)-th chunk, their sums added in thread order.  Bound by the
+// read of the partials (27 * 32 * 32 floats from each of 512 work-groups:
+// 57 MB).  One thread per output and 512 dependent loads each took 108 us
+// whatever the length; RO = 32 keeps 128-byte reads and eight loads in flight
+// per thread (10.3 us, 5.5 TB/s); RO = 8 spreads the short layers (864 values)
+// over 108 work-groups.
+template <int RO>
 __global__ void __launch_bounds__(256)
-k_reduce_chunks(int nchunk, int len, const float* __restrict__ part, float* __restrict__ out) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= len) return;
+k_reduce_chunks(int nchunk, int len, const float* __restrict__ part, float* __restrict__ out,
+                int blen, const float* __restrict__ bpart, float* __restrict__ bout) {
+    constexpr int NG = 256 / RO;
+    __shared__ float sh[256];
+    const int nblk = (len + RO - 1) / RO;                  // work-groups of the weights
+    const bool bias = int(blockIdx.x) >= nblk;
+    const float* src = bias ? bpart : part;
+    const int ln = bias ? blen : len;
+    const int i = (int(blockIdx.x) - (bias ? nblk : 0)) * RO + int(threadIdx.x) % RO;
+    const int g = int(threadIdx.x) / RO;
     float acc = 0.f;
-    for (int c = 0; c < nchunk; ++c) acc += part[size_t(c) * len + i];
-    out[i] = acc;
+    if (i < ln) {
+#pragma unroll 8
+        for (int c = g; c < nchunk; c += NG) acc += src[size_t(c) * ln + i];
+    }
+    sh[threadIdx.x] = acc;
+    __syncthreads();
+    if (g == 0 && i < ln) {
+        for (int k = 1; k < NG; ++k) acc += sh[k * RO + threadIdx.x];
+        (bias ? bout : out)[i] = acc;
+    }
 }
 
 // scaled input of layer 1, rounded to bf16 as the forward uses it, stored as
@@ -1110,6 +1134,20 @@ int launch_wthin(int nb, const float* s1, const __bf16* t32, float* work, int& n
     return 0;
 }
 
+// weight and bias gradients of one layer from its ng partials at work (dW, then db)
+int reduce_partials(int ng, int len, int blen, const float* work, float* dW, float* db,
+                    hipStream_t st) {
+    const float* bw = work + size_t(ng) * len;
+    if (len >= 8192)
+        hipLaunchKernelGGL(k_reduce_chunks<32>, dim3((len + 31) / 32 + (blen + 31) / 32), dim3(256),
+                           0, st, ng, len, work, dW, blen, bw, db);
+    else
+        hipLaunchKernelGGL(k_reduce_chunks<8>, dim3((len + 7) / 8 + (blen + 7) / 8), dim3(256), 0,
+                           st, ng, len, work, dW, blen, bw, db);
+    DGFS_HIP_CHECK(hipGetLastError());
+    return 0;
+}
+
 // thin-layer weight gradient partials (dW then db) at work; ng partials
 int wgrad_thin(int G, bool gc1, int nb, const float* s1, const void* t32, float* work, int& ng,
                hipStream_t st) {
@@ -1199,31 +1237,19 @@ extern "C" int dgfs_closure_backward(const dgfs_closure_t* net, const dgfs_closu
     int ng = 0;
     int rc0 = wgrad_thin(G, true, nb, dOut, A + 5 * a, work, ng, st);
     if (rc0) return rc0;
-    hipLaunchKernelGGL(k_reduce_chunks, dim3((kTaps * kC + 255) / 256), dim3(256), 0, st, ng,
-                       kTaps * kC, work, gr->W4);
-    hipLaunchKernelGGL(k_reduce_chunks, dim3(1), dim3(256), 0, st, ng, 1,
-                       work + size_t(ng) * kTaps * kC, gr->b4);
-    DGFS_HIP_CHECK(hipGetLastError());
+    if ((rc0 = reduce_partials(ng, kTaps * kC, 1, work, gr->W4, gr->b4, st))) return rc0;
     hipLaunchKernelGGL(k_out_bwd, gv, dim3(256), 0, st, G, nvox, dOut, net->W4, A + 4 * a, GA);
     DGFS_HIP_CHECK(hipGetLastError());
     // layer 3: dW3 = dZ3 x Y2, dZ2 = silu'(Z2) convT(dZ3, W3)
     rc0 = wgrad_mid(G, nb, GA, A + 3 * a, work, ng, st);
     if (rc0) return rc0;
-    hipLaunchKernelGGL(k_reduce_chunks, dim3((kTaps * kC * kC + 255) / 256), dim3(256), 0, st, ng,
-                       kTaps * kC * kC, work, gr->W3);
-    hipLaunchKernelGGL(k_reduce_chunks, dim3(1), dim3(256), 0, st, ng, kC,
-                       work + size_t(ng) * kTaps * kC * kC, gr->b3);
-    DGFS_HIP_CHECK(hipGetLastError());
+    if ((rc0 = reduce_partials(ng, kTaps * kC * kC, kC, work, gr->W3, gr->b3, st))) return rc0;
     int rc = dispatch_mid(G, 2, nb, GA, net->W3t, nullptr, A + 2 * a, nullptr, GA + a, st);
     if (rc) return rc;
     // layer 2: dW2 = dZ2 x Y1, dZ1 = silu'(Z1) convT(dZ2, W2)
     rc0 = wgrad_mid(G, nb, GA + a, A + a, work, ng, st);
     if (rc0) return rc0;
-    hipLaunchKernelGGL(k_reduce_chunks, dim3((kTaps * kC * kC + 255) / 256), dim3(256), 0, st, ng,
-                       kTaps * kC * kC, work, gr->W2);
-    hipLaunchKernelGGL(k_reduce_chunks, dim3(1), dim3(256), 0, st, ng, kC,
-                       work + size_t(ng) * kTaps * kC * kC, gr->b2);
-    DGFS_HIP_CHECK(hipGetLastError());
+    if ((rc0 = reduce_partials(ng, kTaps * kC * kC, kC, work, gr->W2, gr->b2, st))) return rc0;
     rc = dispatch_mid(G, 2, nb, GA + a, net->W2t, nullptr, A, nullptr, GA, st);
     if (rc) return rc;
     // layer 1: dW1 = dZ1 x f, db1
@@ -1236,11 +1262,7 @@ extern "C" int dgfs_closure_backward(const dgfs_closure_t* net, const dgfs_closu
     DGFS_HIP_CHECK(hipGetLastError());
     rc0 = wgrad_thin(G, false, nb, fin, GA, work, ng, st);
     if (rc0) return rc0;
-    hipLaunchKernelGGL(k_reduce_chunks, dim3((kTaps * kC + 255) / 256), dim3(256), 0, st, ng,
-                       kTaps * kC, work, gr->W1);
-    hipLaunchKernelGGL(k_reduce_chunks, dim3(1), dim3(256), 0, st, ng, kC,
-                       work + size_t(ng) * kTaps * kC, gr->b1);
-    DGFS_HIP_CHECK(hipGetLastError());
+    if ((rc0 = reduce_partials(ng, kTaps * kC, kC, work, gr->W1, gr->b1, st))) return rc0;
     return 0;
 }
 

@@ -18,9 +18,9 @@
 // as MFMA rows, then a shifted 27-term sum).  Weights are bf16 on the device
 // (W2/W3 packed copies; W1/W4 rounded from the FP32 masters in-kernel).
 // Backward: the 32 -> 32 input gradients reuse the layer-3 kernel with
-// tap-flipped, transposed weights; the thin layers' gradients and all weight
-// gradients run on FP32 VALU with FP32 accumulation, partial weight gradients
-// reduced in a fixed order (deterministic).
+// tap-flipped, transposed weights; weight gradients run on the bf16 (32 -> 32)
+// and FP32 (thin layers) matrix instructions with FP32 accumulation, their
+// partials reduced in a fixed order (deterministic).
 #include "dgfs_common.h"
 #include "dgfs_hip.h"
 
@@ -29,6 +29,7 @@ namespace {
 
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4;
+typedef __attribute__((__vector_size__(16 * sizeof(float)))) float floatx16;
 
 constexpr int kC = 32;          // hidden channels
 constexpr int kTaps = 27;
@@ -803,102 +804,110 @@ k_wgrad_mma(int nb, const __bf16* __restrict__ Gr, const __bf16* __restrict__ X,
     }
 }
 
-// Thin layers (one side has one channel), tiled like k_wgrad_mma:
-//   GC1 = true  (layer 4): out[tap][c] = sum_v s[v] T[v + d][c], s = dOut
-//                          (FP32, the tile), T = Y3 (bf16, planes z-1..z+1)
-//   GC1 = false (layer 1): out[tap][c] = sum_v T[v][c] s[v + d], T = dZ1
-//                          (bf16, the tile), s = scaled input (FP32, halo)
-// and the bias partials (sum of dOut, or of dZ1 per channel).  Thread
-// (c = tid & 31, tq = tid >> 5) owns channel c and taps tq, tq+8, tq+16,
-// tq+24; partials part[wg][tap][c], bpart[wg][32] (GC1: bpart[wg]).
+// Thin layers (one side has one channel) on the FP32 matrix instruction:
+//   out[tap][c] = sum_v T[v][c] s[v + sg d(tap)]
+//   GC1 = true  (layer 4): s = dOut (FP32), T = Y3, sg = -1
+//   GC1 = false (layer 1): s = scaled input (FP32), T = dZ1, sg = +1
+// (s is zero outside the grid), with the bias partials: the sum of dOut, or of
+// dZ1 per channel.  v_mfma_f32_32x32x2f32 with rows = taps (27 of 32), columns
+// = channels and K = two voxels: A lane (tap, k) = s at voxel k shifted by the
+// lane's tap, B lane (c, k) = T[voxel k][c], both one LDS read; row 27 of A is
+// 1, which gives the channel sums.  Products and sums stay FP32.  Tasks are
+// k_wgrad_mma's tiles, a quarter of a tile per wave; the next task's T tile
+// and s halo are loaded into registers while the current one is multiplied.
+// Bound by the two LDS reads per matrix instruction and the tile loads; the
+// vector form (one channel and four taps per thread) took 240 us (layer 4)
+// and 228 us (layer 1) on 16 grids of 32^3, this one 26 and 25 us.
 template <int G, bool GC1>
 __global__ void __launch_bounds__(256)
 k_wgrad_thin(int nb, const float* __restrict__ s1, const __bf16* __restrict__ t32,
              float* __restrict__ part, float* __restrict__ bpart) {
     using W = WgTile<G>;
-    constexpr int HV = 3 * W::HR * W::HX;                   // halo voxels
-    constexpr int TP = GC1 ? HV + 8 : W::TV + 8;            // channel pitch of T (bf16)
-    constexpr int SN = GC1 ? W::TV : HV;                    // scalar field size
-    __shared__ __attribute__((aligned(16))) __bf16 Ts[kC * TP];
-    __shared__ float Ss[SN];
-    const int tid = threadIdx.x, c = tid & 31, tq = tid >> 5;
+    constexpr int HV = 3 * W::HR * W::HX;                   // halo voxels of s
+    constexpr int NTL = W::TV * 4 / 256, NSL = (HV + 255) / 256;   // loads per thread
+    constexpr int SG = GC1 ? -1 : 1;
+    static_assert(W::TV * 4 % 256 == 0 && W::RB % 4 == 0 && W::TV <= 256, "tile split");
+    __shared__ __attribute__((aligned(16))) __bf16 Ts[W::TV * kC];
+    __shared__ float Ss[HV];
+    __shared__ float red[4 * 32 * 32];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int c = lane & 31, kk = lane >> 5;
     const size_t n = size_t(G) * G * G;
     const int ntask = nb * W::NTASK;
-    int toff[4];
-    bool tin[4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        const int tap = tq + 8 * k;
-        tin[k] = tap < kTaps;
-        int dz = 0, dy = 0, dx = 0;
-        if (tin[k]) tap_offset(tap, dz, dy, dx);
-        toff[k] = ((dz + 1) * W::HR + dy + 1) * W::HX + dx + 1;   // halo offset of (0, 0, 0) + d
-    }
-    float acc[4] = {0.f, 0.f, 0.f, 0.f};
+    const int tap = lane & 31;
+    const bool tin = tap < kTaps;
+    int dz = 0, dy = 0, dx = 0;
+    if (tin) tap_offset(tap, dz, dy, dx);
+    const int toff = ((1 + SG * dz) * W::HR + 1 + SG * dy) * W::HX + 1 + SG * dx;
+    const float cst = tap == kTaps ? 1.f : 0.f;             // the row of ones; rows 28.. are 0
+    floatx16 acc = {};
     float bacc = 0.f;
-    for (int task = blockIdx.x; task < ntask; task += gridDim.x) {
+    uint4 tl[NTL];
+    float sl[NSL];
+    auto load = [&](int task) {
         const int b = task / W::NTASK, rr = task - b * W::NTASK;
         const int z = rr / (G / W::RB), y0 = (rr % (G / W::RB)) * W::RB;
-        __syncthreads();
-        if (GC1) {
-            for (int k = tid; k < W::TV; k += 256) {
-                const int y = y0 + k / G, x = k % G;
-                Ss[k] = s1[size_t(b) * n + (size_t(z) * G + y) * G + x];
-            }
-            for (int k = tid; k < HV * 4; k += 256) {
-                const int vox = k >> 2, cg = k & 3;
-                const int pz = vox / (W::HR * W::HX), rem = vox - pz * (W::HR * W::HX);
-                const int r = rem / W::HX, cc = rem - r * W::HX;
-                const int zz = z + pz - 1, y = y0 + r - 1, x = cc - 1;
-                uint4 w = make_uint4(0u, 0u, 0u, 0u);
-                if (zz >= 0 && zz < G && y >= 0 && y < G && x >= 0 && x < G)
-                    w = *reinterpret_cast<const uint4*>(
-                        &t32[(size_t(b) * n + (size_t(zz) * G + y) * G + x) * kC + 8 * cg]);
-                __bf16 h[8];
-                __builtin_memcpy(h, &w, 16);
+        const uint4* tp = reinterpret_cast<const uint4*>(
+            &t32[(size_t(b) * n + (size_t(z) * G + y0) * G) * kC]);
 #pragma unroll
-                for (int e = 0; e < 8; ++e) Ts[(8 * cg + e) * TP + vox] = h[e];
-            }
-        } else {
-            for (int k = tid; k < HV; k += 256) {
-                const int pz = k / (W::HR * W::HX), rem = k - pz * (W::HR * W::HX);
-                const int r = rem / W::HX, cc = rem - r * W::HX;
-                const int zz = z + pz - 1, y = y0 + r - 1, x = cc - 1;
-                float v = 0.f;
-                if (zz >= 0 && zz < G && y >= 0 && y < G && x >= 0 && x < G)
-                    v = s1[size_t(b) * n + (size_t(zz) * G + y) * G + x];
-                Ss[k] = v;
-            }
-            for (int k = tid; k < W::TV * 4; k += 256) {
-                const int tv = k >> 2, cg = k & 3;
-                const int y = y0 + tv / G, x = tv % G;
-                const uint4 w = *reinterpret_cast<const uint4*>(
-                    &t32[(size_t(b) * n + (size_t(z) * G + y) * G + x) * kC + 8 * cg]);
-                __bf16 h[8];
-                __builtin_memcpy(h, &w, 16);
+        for (int k = 0; k < NTL; ++k) tl[k] = tp[tid + 256 * k];
 #pragma unroll
-                for (int e = 0; e < 8; ++e) Ts[(8 * cg + e) * TP + tv] = h[e];
-            }
+        for (int k = 0; k < NSL; ++k) {
+            const int h = tid + 256 * k;
+            const int pz = h / (W::HR * W::HX), rem = h - pz * (W::HR * W::HX);
+            const int r = rem / W::HX, cc = rem - r * W::HX;
+            const int zz = z + pz - 1, y = y0 + r - 1, x = cc - 1;
+            float v = 0.f;
+            if (h < HV && zz >= 0 && zz < G && y >= 0 && y < G && x >= 0 && x < G)
+                v = s1[size_t(b) * n + (size_t(zz) * G + y) * G + x];
+            sl[k] = v;
         }
-        __syncthreads();
-        for (int tv = 0; tv < W::TV; ++tv) {
-            const int r = tv / G, x = tv % G;
-            const int h0 = r * W::HX + x;                 // halo index of (r, x) minus the d offset
-            const float a = GC1 ? Ss[tv] : bf2f(Ts[c * TP + tv]);
-            if (tq == 0) bacc += a;
+    };
+    int task = blockIdx.x;
+    if (task < ntask) load(task);
+    for (; task < ntask; task += gridDim.x) {
+        __syncthreads();                                    // previous task's reads are done
 #pragma unroll
-            for (int k = 0; k < 4; ++k)
-                if (tin[k]) acc[k] += a * (GC1 ? bf2f(Ts[c * TP + h0 + toff[k]]) : Ss[h0 + toff[k]]);
+        for (int k = 0; k < NTL; ++k) reinterpret_cast<uint4*>(Ts)[tid + 256 * k] = tl[k];
+#pragma unroll
+        for (int k = 0; k < NSL; ++k)
+            if (tid + 256 * k < HV) Ss[tid + 256 * k] = sl[k];
+        __syncthreads();
+        if (task + int(gridDim.x) < ntask) load(task + gridDim.x);
+        if (GC1 && tid < W::TV)
+            bacc += Ss[(W::HR + 1 + tid / G) * W::HX + 1 + tid % G];
+        // this wave's voxels: rows (RB / 4) wave .. of the tile
+        const float* sp = Ss + wave * (W::RB / 4) * W::HX + toff + kk;
+        const __bf16* tp = Ts + (wave * (W::TV / 4) + kk) * kC + c;
+#pragma unroll
+        for (int m = 0; m < W::TV / 8; ++m) {
+            constexpr int HX = W::HX;
+            const float a = tin ? sp[(2 * m / G) * HX + (2 * m) % G] : cst;
+            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a, bf2f(tp[2 * m * kC]), acc, 0, 0, 0);
         }
     }
-    float* p = part + size_t(blockIdx.x) * kTaps * kC;
+    // the four waves' sums in wave order; lane holds rows 8 (i / 4) + 4 kk + i % 4, column c
 #pragma unroll
-    for (int k = 0; k < 4; ++k)
-        if (tin[k]) p[(tq + 8 * k) * kC + c] = acc[k];
+    for (int i = 0; i < 16; ++i)
+        red[(wave * 32 + 8 * (i / 4) + 4 * kk + i % 4) * 32 + c] = acc[i];
+    __syncthreads();
+    float* p = part + size_t(blockIdx.x) * kTaps * kC;
+    for (int k = tid; k < (kTaps + 1) * kC; k += 256) {
+        const float v = ((red[k] + red[1024 + k]) + red[2048 + k]) + red[3072 + k];
+        if (k < kTaps * kC)
+            p[k] = v;
+        else if (!GC1)
+            bpart[size_t(blockIdx.x) * kC + k - kTaps * kC] = v;
+    }
     if (GC1) {
-        if (tid == 0) bpart[blockIdx.x] = bacc;           // the same sum in every channel lane
-    } else if (tq == 0) {
-        bpart[size_t(blockIdx.x) * kC + c] = bacc;
+        __syncthreads();
+        red[tid] = bacc;
+        __syncthreads();
+        if (tid == 0) {
+            float v = 0.f;
+            for (int k = 0; k < W::TV; ++k) v += red[k];
+            bpart[blockIdx.x] = v;
+        }
     }
 }
 

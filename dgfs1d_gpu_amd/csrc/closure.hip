@@ -664,17 +664,24 @@ k_out_bwd(int G, long nvox, const float* __restrict__ dOut, const float* __restr
 // ------------------------------------------------ weight gradients
 // ------------------------------------------- 32 -> 32 weight gradient, MFMA
 // dW[tap][co][ci] = sum_v Gr[v][co] X[v + d(tap)][ci] and db[co] = sum_v Gr[v][co]
-// over [nb][G^3][32] bf16 tensors.  A task is RB rows x G columns of one
-// plane z of one slice; persistent work-groups stage, per task, the task's
-// Gr tile and X planes z-1..z+1 (rows y0-1..y0+RB, zero halo) channel-major
-// in LDS: GT[co][voxel] and XT[ci][plane][row][column].
-// v_mfma_f32_16x16x32_bf16 with rows = co (16 jc + ..), columns = ci
-// (16 ic + ..) and K = 32 voxels of the tile: A lane (li, kq) =
-// GT[16 jc + li][k0 + 8kq .. +7] (one 16 B read, shared by every tap), B lane
-// (li, kq) = X at the same 8 voxels shifted by d(tap), channel 16 ic + li
-// (eight 2 B reads).  Wave w accumulates taps w, w+4, ... in FP32 over all of
-// its tasks; each work-group writes one partial dW and db (reduced afterwards
-// in a fixed order).
+// over [nb][G^3][32] bf16 tensors.  A task is RB rows x G columns x zc planes
+// of one slice; persistent work-groups march through a task's planes with the
+// X planes z-1..z+1 (rows y0-1..y0+RB) in a channel-major LDS ring
+// XT[ci][slot][row][column] and the plane's Gr tile in GT[co][voxel]: each
+// plane is fetched once per task, the next one into registers while the
+// current one is multiplied.  v_mfma_f32_16x16x32_bf16 with rows = co
+// (16 jc + ..), columns = ci (16 ic + ..) and K = 32 voxels of the tile: A lane
+// (li, kq) = GT[16 jc + li][k0 + 8kq .. +7] (one 16 B read, shared by every
+// tap), B lane (li, kq) = X at the same 8 voxels shifted by d(tap), channel
+// 16 ic + li.  The three dx taps of a (dz, dy) come from one aligned 16 B read
+// and the 4 B on each side of it, shifted by v_alignbit.  The 18 (dz, dy, ic)
+// are dealt out to the four waves (5, 5, 4, 4), accumulated in FP32 over all
+// of a wave's tasks; each work-group writes one partial dW and db (reduced
+// afterwards in a fixed order).
+// Bound by LDS: three reads per 12 matrix instructions and the transposing
+// writes.  With eight 2 B reads per shifted fragment and all three planes
+// staged for every plane of output it took 138 us on 16 grids of 32^3, this
+// form 89 us (330 TFLOP/s).
 template <int G>
 struct WgTile {
     static constexpr int RB = G == 16 ? 8 : 4;             // rows per task
@@ -682,97 +689,147 @@ struct WgTile {
     static constexpr int NK = TV / 32;                    // K chunks
     static constexpr int HR = RB + 2, HX = G + 2;
     static constexpr int GTP = TV + 8;                    // GT row pitch (bf16)
-    static constexpr int XTP = 3 * HR * HX + 8;           // XT channel pitch (bf16)
-    static constexpr int NTASK = G * (G / RB);            // tasks per slice
-    static_assert(TV % 32 == 0 && G % RB == 0, "tile");
+    static constexpr int NTASK = G * (G / RB);            // tiles (of one plane) per slice
+    // XT: rows of G columns behind 8 zero columns (the left neighbour of
+    // column 0; the first of the next row's is the right neighbour of column
+    // G - 1), so that columns x % 8 == 0 are 16 B aligned; the channel pitch
+    // is 96 elements modulo 128, which spreads a fragment's 16 channels x 64 B
+    // over all banks
+    static constexpr int XR = G + 8, XPL = HR * XR;        // row, plane
+    static constexpr int XTP = (3 * XPL + 8 - 96 + 127) / 128 * 128 + 96;
+    static constexpr int CG = G / 4;                      // column groups of a row
+    static constexpr int NXU = HR * CG * 4, NGU = RB * CG * 4;   // staging units of a plane
+    static_assert(TV % 32 == 0 && G % RB == 0 && G % 8 == 0, "tile");
 };
 
 template <int G>
 __global__ void __launch_bounds__(256)
-k_wgrad_mma(int nb, const __bf16* __restrict__ Gr, const __bf16* __restrict__ X,
+k_wgrad_mma(int nb, int zc, const __bf16* __restrict__ Gr, const __bf16* __restrict__ X,
             float* __restrict__ part, float* __restrict__ bpart) {
     using W = WgTile<G>;
-    constexpr int MT = (kTaps + 3) / 4;                   // taps per wave
+    constexpr int NU = 18, MU = 5;                        // (dz, dy, ic) units, per wave
+    constexpr int NL = (W::NXU + W::NGU + 255) / 256;     // staging units per thread
     __shared__ __attribute__((aligned(16))) __bf16 GT[kC * W::GTP];
     __shared__ __attribute__((aligned(16))) __bf16 XT[kC * W::XTP];
-    __shared__ float sb[256 * 8];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, li = lane & 15, kq = lane >> 4;
+    const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, kq = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const size_t n = size_t(G) * G * G;
-    const int ntask = nb * W::NTASK;
+    constexpr int YB = G / W::RB;
+    const int per = YB * (G / zc), ntask = nb * per;
     const int cg = tid & 3;                               // channel group of this thread's loads
     float bsum[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    floatx4 acc[MT][2][2];
+    floatx4 acc[MU][3][2];
 #pragma unroll
-    for (int m = 0; m < MT; ++m)
+    for (int m = 0; m < MU; ++m)
 #pragma unroll
-        for (int jc = 0; jc < 2; ++jc)
+        for (int d = 0; d < 3; ++d)
 #pragma unroll
-            for (int ic = 0; ic < 2; ++ic) acc[m][jc][ic] = floatx4{0.f, 0.f, 0.f, 0.f};
-    for (int task = blockIdx.x; task < ntask; task += gridDim.x) {
-        const int b = task / W::NTASK, rr = task - b * W::NTASK;
-        const int z = rr / (G / W::RB), y0 = (rr % (G / W::RB)) * W::RB;
-        const __bf16* Gb = Gr + size_t(b) * n * kC;
-        const __bf16* Xb = X + size_t(b) * n * kC;
-        __syncthreads();                                  // previous task's reads are done
-        // Gr tile, transposed; bias partial sums (this thread's 8 channels)
-        for (int k = tid; k < W::TV * 4; k += 256) {
-            const int tv = k >> 2;
-            const int y = y0 + tv / G, x = tv % G;
-            const uint4 w = *reinterpret_cast<const uint4*>(
-                &Gb[((size_t(z) * G + y) * G + x) * kC + 8 * cg]);
-            __bf16 h[8];
-            __builtin_memcpy(h, &w, 16);
+            for (int jc = 0; jc < 2; ++jc) acc[m][d][jc] = floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int k = tid; k < kC * W::XTP / 8; k += 256)      // the zero columns stay zero
+        reinterpret_cast<uint4*>(XT)[k] = make_uint4(0u, 0u, 0u, 0u);
+    // a thread's staging units of step q: four columns x 8 channels of X plane
+    // q (rows y0 - 1 ..) or of Gr plane q - 1
+    uint4 st[NL][4];
+    auto load = [&](const __bf16* Gb, const __bf16* Xb, int y0, int z0, int q) {
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                GT[(8 * cg + e) * W::GTP + tv] = h[e];
-                bsum[e] += bf2f(h[e]);
+        for (int l = 0; l < NL; ++l) {
+            const int u = tid + 256 * l;
+            const bool isx = u < W::NXU;
+            const int w = (isx ? u : u - W::NXU) >> 2;
+            const int r = w / W::CG, x = 4 * (w - r * W::CG);
+            const int y = isx ? y0 + r - 1 : y0 + r, z = isx ? q : q - 1;
+            const bool in = u < W::NXU + W::NGU && z >= (isx ? 0 : z0) && z < G && y >= 0 && y < G;
+            const uint4* p = reinterpret_cast<const uint4*>(
+                (isx ? Xb : Gb) + ((size_t(in ? z : 0) * G + (in ? y : 0)) * G + x) * kC + 8 * cg);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) st[l][k] = in ? p[4 * k] : make_uint4(0u, 0u, 0u, 0u);
+        }
+    };
+    auto store = [&](int q) {
+        const int slot = (q + 3) % 3;
+#pragma unroll
+        for (int l = 0; l < NL; ++l) {
+            const int u = tid + 256 * l;
+            if (u >= W::NXU + W::NGU) break;
+            const bool isx = u < W::NXU;
+            const int w = (isx ? u : u - W::NXU) >> 2;
+            const int r = w / W::CG, x = 4 * (w - r * W::CG);
+            unsigned v[4][4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                v[k][0] = st[l][k].x; v[k][1] = st[l][k].y;
+                v[k][2] = st[l][k].z; v[k][3] = st[l][k].w;
+            }
+            __bf16* dst = isx ? XT + 8 * cg * W::XTP + slot * W::XPL + r * W::XR + 8 + x
+                              : GT + 8 * cg * W::GTP + r * G + x;
+            const int pitch = isx ? W::XTP : W::GTP;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {                 // channels 2e, 2e + 1 of the group
+                uint2 lo, hi;
+                lo.x = __builtin_amdgcn_perm(v[1][e], v[0][e], 0x05040100u);
+                lo.y = __builtin_amdgcn_perm(v[3][e], v[2][e], 0x05040100u);
+                hi.x = __builtin_amdgcn_perm(v[1][e], v[0][e], 0x07060302u);
+                hi.y = __builtin_amdgcn_perm(v[3][e], v[2][e], 0x07060302u);
+                *reinterpret_cast<uint2*>(dst + 2 * e * pitch) = lo;
+                *reinterpret_cast<uint2*>(dst + (2 * e + 1) * pitch) = hi;
+                if (!isx) {
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        bsum[2 * e] += __builtin_bit_cast(float, v[k][e] << 16);
+                        bsum[2 * e + 1] += __builtin_bit_cast(float, v[k][e] & 0xffff0000u);
+                    }
+                }
             }
         }
-        // X planes z-1..z+1 with zero halo, transposed
-        for (int k = tid; k < 3 * W::HR * W::HX * 4; k += 256) {
-            const int vox = k >> 2;
-            const int pz = vox / (W::HR * W::HX), rem = vox - pz * (W::HR * W::HX);
-            const int r = rem / W::HX, c = rem - r * W::HX;
-            const int zz = z + pz - 1, y = y0 + r - 1, x = c - 1;
-            uint4 w = make_uint4(0u, 0u, 0u, 0u);
-            if (zz >= 0 && zz < G && y >= 0 && y < G && x >= 0 && x < G)
-                w = *reinterpret_cast<const uint4*>(
-                    &Xb[((size_t(zz) * G + y) * G + x) * kC + 8 * cg]);
-            __bf16 h[8];
-            __builtin_memcpy(h, &w, 16);
+    };
+    for (int task = blockIdx.x; task < ntask; task += gridDim.x) {
+        const int b = task / per, rr = task - b * per;
+        const int z0 = (rr / YB) * zc, y0 = (rr % YB) * W::RB;
+        const __bf16* Gb = Gr + size_t(b) * n * kC;
+        const __bf16* Xb = X + size_t(b) * n * kC;
+        load(Gb, Xb, y0, z0, z0 - 1);
+        for (int q = z0 - 1; q <= z0 + zc; ++q) {
+            __syncthreads();                              // the previous plane's reads are done
+            store(q);
+            __syncthreads();
+            if (q < z0 + zc) load(Gb, Xb, y0, z0, q + 1);
+            if (q <= z0) continue;
+            const int z = q - 1;
+            bf16x8 a[W::NK][2];
 #pragma unroll
-            for (int e = 0; e < 8; ++e) XT[(8 * cg + e) * W::XTP + vox] = h[e];
-        }
-        __syncthreads();
-        bf16x8 a[W::NK][2];
+            for (int kc = 0; kc < W::NK; ++kc)
 #pragma unroll
-        for (int kc = 0; kc < W::NK; ++kc)
+                for (int jc = 0; jc < 2; ++jc)
+                    a[kc][jc] = *reinterpret_cast<const bf16x8*>(
+                        &GT[(16 * jc + li) * W::GTP + kc * 32 + 8 * kq]);
 #pragma unroll
-            for (int jc = 0; jc < 2; ++jc)
-                a[kc][jc] = *reinterpret_cast<const bf16x8*>(
-                    &GT[(16 * jc + li) * W::GTP + kc * 32 + 8 * kq]);
+            for (int m = 0; m < MU; ++m) {
+                const int u = wave + 4 * m;
+                if (u >= NU) break;
+                const int g = u >> 1, ic = u & 1, dz = g / 3 - 1, dy = g % 3 - 1;
+                const __bf16* xb = XT + (16 * ic + li) * W::XTP + ((z + dz + 3) % 3) * W::XPL +
+                                   (dy + 1) * W::XR + 8;
 #pragma unroll
-        for (int m = 0; m < MT; ++m) {
-            const int tap = wave + 4 * m;
-            if (tap >= kTaps) break;
-            int dz, dy, dx;
-            tap_offset(tap, dz, dy, dx);
+                for (int kc = 0; kc < W::NK; ++kc) {
+                    // the lane's 8 voxels lie in one row: tile voxel kc*32 + 8kq + e
+                    const int tv = kc * 32 + 8 * kq;
+                    const __bf16* src = xb + (tv / G) * W::XR + tv % G;
+                    const uint4 d = *reinterpret_cast<const uint4*>(src);
+                    const unsigned dm = *reinterpret_cast<const unsigned*>(src - 2);
+                    const unsigned dp = *reinterpret_cast<const unsigned*>(src + 8);
+                    const unsigned s1 = __builtin_amdgcn_alignbit(d.y, d.x, 16),
+                                   s2 = __builtin_amdgcn_alignbit(d.z, d.y, 16),
+                                   s3 = __builtin_amdgcn_alignbit(d.w, d.z, 16);
+                    const uint4 t[3] = {
+                        make_uint4(__builtin_amdgcn_alignbit(d.x, dm, 16), s1, s2, s3), d,
+                        make_uint4(s1, s2, s3, __builtin_amdgcn_alignbit(dp, d.w, 16))};
 #pragma unroll
-            for (int kc = 0; kc < W::NK; ++kc) {
-                // the lane's 8 voxels lie in one row: tile voxel kc*32 + 8kq + e
-                const int tv = kc * 32 + 8 * kq;
-                const int r = tv / G, x = tv % G;
-                const int off = ((dz + 1) * W::HR + r + dy + 1) * W::HX + x + dx + 1;
+                    for (int dx = 0; dx < 3; ++dx)
 #pragma unroll
-                for (int ic = 0; ic < 2; ++ic) {
-                    const __bf16* src = &XT[(16 * ic + li) * W::XTP + off];
-                    bf16x8 bv;
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) bv[e] = src[e];
-#pragma unroll
-                    for (int jc = 0; jc < 2; ++jc)
-                        acc[m][jc][ic] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                            a[kc][jc], bv, acc[m][jc][ic], 0, 0, 0);
+                        for (int jc = 0; jc < 2; ++jc)
+                            acc[m][dx][jc] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                                a[kc][jc], __builtin_bit_cast(bf16x8, t[dx]), acc[m][dx][jc], 0, 0,
+                                0);
                 }
             }
         }
@@ -780,19 +837,21 @@ k_wgrad_mma(int nb, const __bf16* __restrict__ Gr, const __bf16* __restrict__ X,
     // partial dW of this work-group: lane holds co = 16 jc + 4 kq + i, ci = 16 ic + li
     float* p = part + size_t(blockIdx.x) * kTaps * kC * kC;
 #pragma unroll
-    for (int m = 0; m < MT; ++m) {
-        const int tap = wave + 4 * m;
-        if (tap >= kTaps) break;
+    for (int m = 0; m < MU; ++m) {
+        const int u = wave + 4 * m;
+        if (u >= NU) break;
 #pragma unroll
-        for (int jc = 0; jc < 2; ++jc)
+        for (int dx = 0; dx < 3; ++dx)
 #pragma unroll
-            for (int ic = 0; ic < 2; ++ic)
+            for (int jc = 0; jc < 2; ++jc)
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
-                    p[(size_t(tap) * kC + 16 * jc + 4 * kq + i) * kC + 16 * ic + li] =
-                        acc[m][jc][ic][i];
+                    p[(size_t(3 * (u >> 1) + dx) * kC + 16 * jc + 4 * kq + i) * kC +
+                      16 * (u & 1) + li] = acc[m][dx][jc][i];
     }
     // bias partial: threads with the same channel group, in a fixed order
+    __syncthreads();
+    float* sb = reinterpret_cast<float*>(XT);
 #pragma unroll
     for (int e = 0; e < 8; ++e) sb[tid * 8 + e] = bsum[e];
     __syncthreads();
@@ -1120,11 +1179,15 @@ int launch_forward(const dgfs_closure_t* net, int nb, const T* u, const int* src
 // work (dW partials, then db partials); ng receives the number of partials
 template <int G>
 int launch_wgrad(int nb, const __bf16* g, const __bf16* x, float* work, int& ng, hipStream_t st) {
-    const int ntask = nb * WgTile<G>::NTASK;
     int cap = 2 * cu_count();
     if (cap > kWgradMaxGridDev) cap = kWgradMaxGridDev;
+    // planes per task: eight fetch 10 planes of X for 8 of output (one plane
+    // per task would fetch 3 for 1), fewer where that leaves work-groups idle
+    int zc = 8;
+    while (zc > 1 && nb * (G / WgTile<G>::RB) * (G / zc) < cap) zc /= 2;
+    const int ntask = nb * (G / WgTile<G>::RB) * (G / zc);
     ng = ntask < cap ? ntask : cap;
-    hipLaunchKernelGGL((k_wgrad_mma<G>), dim3(ng), dim3(256), 0, st, nb, g, x, work,
+    hipLaunchKernelGGL((k_wgrad_mma<G>), dim3(ng), dim3(256), 0, st, nb, zc, g, x, work,
                        work + size_t(ng) * kTaps * kC * kC);
     DGFS_HIP_CHECK(hipGetLastError());
     return 0;

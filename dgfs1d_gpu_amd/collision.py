@@ -257,6 +257,13 @@ class BiCollisionPlan:
         n = t['K'] * t['Ne'] * self.n
         if min(up.numel(), uq.numel(), Q.numel()) < n:
             raise ValueError('collision operands smaller than K*Ne*Nv')
+        if t['fg_same'] and up.data_ptr() == uq.data_ptr():
+            # a species with itself, f = g in every task
+            _lib.check(_lib.lib().dgfs_bi_collide_like(
+                self._h, _lib.ptr(up), _lib.ptr(Q), t['K'], t['Ne'], t['ntask'],
+                _lib.ptr(t['nterm']), _lib.ptr(t['slice']), _lib.ptr(t['coef']), t['ngroup'],
+                _lib.ptr(t['gstart']), _lib.ptr(t['gslice']), _lib.stream_ptr(stream)))
+            return
         _lib.check(_lib.lib().dgfs_bi_collide(
             self._h, _lib.ptr(up), _lib.ptr(uq), _lib.ptr(Q), t['K'], t['Ne'], t['ntask'],
             _lib.ptr(t['nterm']), _lib.ptr(t['slice']), _lib.ptr(t['coef']), t['ngroup'],

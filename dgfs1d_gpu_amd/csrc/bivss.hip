@@ -67,52 +67,89 @@ k_bi_ctab(int N, int Nrho, int Mpre, const double* __restrict__ fac,
     ctab[k] = mk(T(cr), T(ci));
 }
 
-template <typename T>
-static int bi_dispatch(BiPlan* pl, const void* up, const void* uq, void* Q, TaskView tv,
-                       int ntask, int ngroup, const int* gs, const int* gsl, hipStream_t st) {
-    switch (pl->N) {
-        case 4: return bi_launch<T, 4>(pl, up, uq, Q, tv, ntask, ngroup, gs, gsl, st);
-        case 6: return bi_launch<T, 6>(pl, up, uq, Q, tv, ntask, ngroup, gs, gsl, st);
-        case 8: return bi_launch<T, 8>(pl, up, uq, Q, tv, ntask, ngroup, gs, gsl, st);
-        case 12: return bi_launch<T, 12>(pl, up, uq, Q, tv, ntask, ngroup, gs, gsl, st);
-        case 16: return bi_launch<T, 16>(pl, up, uq, Q, tv, ntask, ngroup, gs, gsl, st);
-        case 20: return bi_launch<T, 20>(pl, up, uq, Q, tv, ntask, ngroup, gs, gsl, st);
-        case 24: return bi_launch<T, 24>(pl, up, uq, Q, tv, ntask, ngroup, gs, gsl, st);
-        case 32: return bi_launch<T, 32>(pl, up, uq, Q, tv, ntask, ngroup, gs, gsl, st);
+// f(std::integral_constant<int, N>) for the plan's grid; N = 48 is FP32 only
+template <typename T, typename Fn>
+static int bi_for_grid(int N, Fn&& f) {
+    switch (N) {
+        case 4: return f(std::integral_constant<int, 4>{});
+        case 6: return f(std::integral_constant<int, 6>{});
+        case 8: return f(std::integral_constant<int, 8>{});
+        case 12: return f(std::integral_constant<int, 12>{});
+        case 16: return f(std::integral_constant<int, 16>{});
+        case 20: return f(std::integral_constant<int, 20>{});
+        case 24: return f(std::integral_constant<int, 24>{});
+        case 32: return f(std::integral_constant<int, 32>{});
         case 48:
-            if constexpr (sizeof(T) == 4)
-                return bi_launch<T, 48>(pl, up, uq, Q, tv, ntask, ngroup, gs, gsl, st);
+            if constexpr (sizeof(T) == 4) return f(std::integral_constant<int, 48>{});
             break;
         default: break;
     }
-    set_error("bi_collide: unsupported velocity grid N=%d", pl->N);
+    set_error("bi_collide: unsupported velocity grid N=%d", N);
     return 2;
 }
 
 static void bi_free(BiPlan* pl) {
-    for (void* p : {pl->phase, pl->wtab, pl->ctab, pl->Fhat, pl->Iw, pl->acc, pl->H, pl->Gp})
+    for (void* p : {pl->phase, pl->wtab, pl->wspec, pl->ctab, pl->Fhat, pl->Iw, pl->Y, pl->nyq,
+                    pl->acc, pl->H, pl->norm, pl->Gp})
         if (p) (void)hipFree(p);
     delete pl;
 }
 
-// largest number of xy groups of the plane stage (bi_xgroups_max<N>)
-static int bi_gp_groups(int N, int NXY) {
-    switch (N) {
-        case 4: return bi_xgroups_max<4>(NXY);
-        case 6: return bi_xgroups_max<6>(NXY);
-        case 8: return bi_xgroups_max<8>(NXY);
-        case 12: return bi_xgroups_max<12>(NXY);
-        case 16: return bi_xgroups_max<16>(NXY);
-        case 20: return bi_xgroups_max<20>(NXY);
-        case 24: return bi_xgroups_max<24>(NXY);
-        case 32: return bi_xgroups_max<32>(NXY);
-        default: return bi_xgroups_max<48>(NXY);
+// element counts of a grid's device arrays
+struct BiSizes {
+    size_t wtab = 0, wspec = 0;             // weight tables
+    size_t Y = 0, nyq = 0, acc = 0;         // per task
+    size_t group = 0;                       // one group's partial G^ of a task
+    int groups = 1;                         // groups that Gp holds
+    size_t ctab = 0;                        // c_pq
+};
+template <int N>
+static BiSizes bi_sizes(bool stream, int NXY, int NU) {
+    using Gm = BiGeo<N>;
+    BiSizes z;
+    if (stream) {
+        z.wtab = size_t(NU) * N * Gm::NPT;
+        z.wspec = size_t(NU) * Gm::NPH;
+        z.Y = size_t(NXY) * Gm::n;
+        z.nyq = size_t(NXY) * 3 * Gm::NN;
+        z.acc = size_t(NXY) * size_t(N + kBiXSMax) * Gm::NPT;
+        z.group = size_t(N) * Gm::NPT;
+        z.groups = NU < 64 ? NU : 64;
+        z.ctab = size_t(N) * Gm::NPH;
+    } else {
+        z.wtab = z.acc = size_t(NXY) * Gm::n;
+        z.group = Gm::n;
+        z.groups = bi_xgroups_max<N>(NXY);
+        z.ctab = Gm::n;
     }
+    return z;
+}
+static BiSizes bi_sizes_of(const BiPlan* pl) {
+    BiSizes z;
+    const int NXY = pl->Nrho * pl->M;
+    (void)bi_for_grid<float>(pl->N, [&](auto n) {
+        z = bi_sizes<int(n)>(pl->stream, NXY, pl->antipodal ? NXY / 2 : NXY);
+        return 0;
+    });
+    return z;
+}
+
+// opp[i] = the index of the exactly opposite point of a rule, -1 without one
+static std::vector<int> opposite(const double* p, int n) {
+    std::vector<int> o(n, -1);
+    for (int i = 0; i < n; ++i)
+        for (int j = 0; j < n && o[i] < 0; ++j)
+            if (j != i && p[3 * j] == -p[3 * i] && p[3 * j + 1] == -p[3 * i + 1] &&
+                p[3 * j + 2] == -p[3 * i + 2])
+                o[i] = j;
+    for (int i = 0; i < n; ++i)             // repeated points pair up one to one or not at all
+        if (o[i] >= 0 && o[o[i]] != i) o[i] = -1;
+    return o;
 }
 
 // scratch budget of the gain products: tasks are processed in chunks whose
 // [chunk][Nrho*M][n] complex products fit in it
-constexpr size_t kBiAccBudget = size_t(2) << 30;
+constexpr size_t kBiAccBudget = size_t(4) << 30;
 
 }  // namespace dgfs
 
@@ -163,15 +200,32 @@ extern "C" int dgfs_bi_collision_plan_create(int N, int M, int Nrho, double L, c
         wc[x] = qw[x] * sw * fb;
     }
     const double mqf = mq / (mp + mq), mpf = mp / (mp + mq);
+    const bool stream =
+        dgfs::bi_streams(N) &&
+        ((dtype == DGFS_F64 ? dgfs::pick_split<double>(N) : dgfs::pick_split<float>(N)) > 1 ||
+         size_t(ntask_max) * NXY * n * cs >= dgfs::kBiStreamBytes);
+    // the direction of the j-th product of a radius: opposite points next to
+    // each other where both rules are antipodally symmetric
+    std::vector<int> ylist;
+    const std::vector<int> oy = dgfs::opposite(sz, M), op = dgfs::opposite(szpre, Mpre);
+    bool antipodal = stream && M % 2 == 0;
+    for (int v : oy) antipodal = antipodal && v >= 0;
+    for (int v : op) antipodal = antipodal && v >= 0;
+    for (int y = 0; y < M; ++y) {
+        if (antipodal && oy[y] < y) continue;
+        ylist.push_back(y);
+        if (antipodal) ylist.push_back(oy[y]);
+    }
     std::vector<double> ph(size_t(NXY) * 2 * 3 * N * 2);
     for (int x = 0; x < Nrho; ++x)
-        for (int y = 0; y < M; ++y)
+        for (int j = 0; j < M; ++j)
             for (int side = 0; side < 2; ++side)
                 for (int ax = 0; ax < 3; ++ax)
                     for (int i = 0; i < N; ++i) {
                         const double l = i < N / 2 ? double(i) : double(i - N);
-                        const double th = (side == 0 ? mqf : -mpf) * fac[x] * sz[3 * y + ax] * l;
-                        const size_t o = ((((size_t(x) * M + y) * 2 + side) * 3 + ax) * N + i) * 2;
+                        const double th =
+                            (side == 0 ? mqf : -mpf) * fac[x] * sz[3 * ylist[j] + ax] * l;
+                        const size_t o = ((((size_t(x) * M + j) * 2 + side) * 3 + ax) * N + i) * 2;
                         ph[o] = std::cos(th);
                         ph[o + 1] = std::sin(th);
                     }
@@ -179,9 +233,11 @@ extern "C" int dgfs_bi_collision_plan_create(int N, int M, int Nrho, double L, c
     auto* pl = new BiPlan();
     pl->N = N; pl->M = M; pl->Nrho = Nrho; pl->Mpre = Mpre; pl->dtype = dtype;
     pl->ntask_max = ntask_max; pl->prefac = prefac; pl->mp = mp; pl->mq = mq; pl->n = n;
-    const bool slabs = (dtype == DGFS_F64 ? dgfs::pick_split<double>(N)
-                                          : dgfs::pick_split<float>(N)) > 1;
-    const size_t per_task = size_t(NXY) * n * cs * (slabs ? 2 : 1);
+    pl->stream = stream;
+    pl->antipodal = antipodal;
+    const dgfs::BiSizes sizes = dgfs::bi_sizes_of(pl);
+    pl->xg_max = sizes.groups;
+    const size_t per_task = (sizes.Y + sizes.nyq + sizes.acc) * cs;
     size_t budget = dgfs::kBiAccBudget;
     if (const char* mb = std::getenv("DGFS_BI_SCRATCH_MB")) {
         const long v = std::atol(mb);
@@ -193,9 +249,9 @@ extern "C" int dgfs_bi_collision_plan_create(int N, int M, int Nrho, double L, c
     pl->chunk = int(chunk);
 
     void *d_fac = nullptr, *d_wx = nullptr, *d_wc = nullptr, *d_sp = nullptr, *d_B = nullptr,
-         *d_Bs = nullptr;
+         *d_Bs = nullptr, *d_yl = nullptr;
     auto fail = [&](int rc) {
-        for (void* p : {d_fac, d_wx, d_wc, d_sp, d_B, d_Bs})
+        for (void* p : {d_fac, d_wx, d_wc, d_sp, d_B, d_Bs, d_yl})
             if (p) (void)hipFree(p);
         dgfs::bi_free(pl);
         return rc;
@@ -206,18 +262,25 @@ extern "C" int dgfs_bi_collision_plan_create(int N, int M, int Nrho, double L, c
     };
     if (!up64(&d_fac, fac.data(), Nrho) || !up64(&d_wx, wx.data(), Nrho) ||
         !up64(&d_wc, wc.data(), Nrho) || !up64(&d_sp, szpre, size_t(Mpre) * 3) ||
-        !up64(&d_B, Bt.data(), Bt.size()) || !up64(&d_Bs, Bsum.data(), Mpre)) {
+        !up64(&d_B, Bt.data(), Bt.size()) || !up64(&d_Bs, Bsum.data(), Mpre) ||
+        hipMalloc(&d_yl, size_t(M) * sizeof(int)) != hipSuccess ||
+        hipMemcpy(d_yl, ylist.data(), size_t(M) * sizeof(int), hipMemcpyHostToDevice) !=
+            hipSuccess) {
         dgfs::set_error("bi_collision_plan_create: table upload failed");
         return fail(1);
     }
     if (hipMalloc(&pl->phase, ph.size() / 2 * cs) != hipSuccess ||
-        hipMalloc(&pl->wtab, size_t(NXY) * n * cs) != hipSuccess ||
-        hipMalloc(&pl->ctab, n * cs) != hipSuccess ||
+        hipMalloc(&pl->wtab, sizes.wtab * cs) != hipSuccess ||
+        (sizes.wspec && hipMalloc(&pl->wspec, sizes.wspec * cs) != hipSuccess) ||
+        (sizes.Y && hipMalloc(&pl->Y, chunk * sizes.Y * cs) != hipSuccess) ||
+        (sizes.nyq && hipMalloc(&pl->nyq, chunk * sizes.nyq * cs) != hipSuccess) ||
+        hipMalloc(&pl->ctab, sizes.ctab * cs) != hipSuccess ||
         hipMalloc(&pl->Fhat, chunk * 2 * n * cs) != hipSuccess ||
         hipMalloc(&pl->Iw, chunk * 2 * n * cs) != hipSuccess ||
-        hipMalloc(&pl->acc, chunk * per_task) != hipSuccess ||
+        hipMalloc(&pl->norm, chunk * 2 * dgfs::bi_norm_blocks(N) * sizeof(double)) != hipSuccess ||
+        hipMalloc(&pl->acc, chunk * sizes.acc * cs) != hipSuccess ||
         hipMalloc(&pl->H, size_t(ntask_max) * 2 * n * cs) != hipSuccess ||
-        hipMalloc(&pl->Gp, chunk * size_t(dgfs::bi_gp_groups(N, NXY)) * n * cs) != hipSuccess) {
+        hipMalloc(&pl->Gp, chunk * size_t(sizes.groups) * sizes.group * cs) != hipSuccess) {
         dgfs::set_error("bi_collision_plan_create: allocation failed");
         return fail(1);
     }
@@ -233,27 +296,33 @@ extern "C" int dgfs_bi_collision_plan_create(int N, int M, int Nrho, double L, c
             return fail(1);
         }
     }
-    const long nb = (long(NXY) * long(n) + 255) / 256, nc = (long(n) + 255) / 256;
-    if (es == 8) {
-        hipLaunchKernelGGL(dgfs::k_bi_btab<double>, dim3(nb), dim3(256), 0, 0, N, M, NXY, Mpre,
-                           (const double*)d_fac, (const double*)d_wx, (const double*)d_sp,
-                           (const double*)d_B, mqf, (dgfs::cplx<double>*)pl->wtab);
-        hipLaunchKernelGGL(dgfs::k_bi_ctab<double>, dim3(nc), dim3(256), 0, 0, N, Nrho, Mpre,
-                           (const double*)d_fac, (const double*)d_wc, (const double*)d_sp,
-                           (const double*)d_Bs, (dgfs::cplx<double>*)pl->ctab);
-    } else {
-        hipLaunchKernelGGL(dgfs::k_bi_btab<float>, dim3(nb), dim3(256), 0, 0, N, M, NXY, Mpre,
-                           (const double*)d_fac, (const double*)d_wx, (const double*)d_sp,
-                           (const double*)d_B, mqf, (dgfs::cplx<float>*)pl->wtab);
-        hipLaunchKernelGGL(dgfs::k_bi_ctab<float>, dim3(nc), dim3(256), 0, 0, N, Nrho, Mpre,
-                           (const double*)d_fac, (const double*)d_wc, (const double*)d_sp,
-                           (const double*)d_Bs, (dgfs::cplx<float>*)pl->ctab);
+    auto tables = [&](auto zero) -> int {
+        using T = decltype(zero);
+        if (pl->stream)
+            return dgfs::bi_for_grid<T>(N, [&](auto g) {
+                return dgfs::bi_stream_tables<T, int(g)>(
+                    pl, (const int*)d_yl, (const double*)d_fac, (const double*)d_wx,
+                    (const double*)d_sp, (const double*)d_B, (const double*)d_wc,
+                    (const double*)d_Bs, mqf);
+            });
+        hipLaunchKernelGGL(dgfs::k_bi_ctab<T>, dim3((long(n) + 255) / 256), dim3(256), 0, 0, N, Nrho,
+                           Mpre, (const double*)d_fac, (const double*)d_wc, (const double*)d_sp,
+                           (const double*)d_Bs, (dgfs::cplx<T>*)pl->ctab);
+        hipLaunchKernelGGL(dgfs::k_bi_btab<T>, dim3((long(NXY) * long(n) + 255) / 256), dim3(256), 0,
+                           0, N, M, NXY, Mpre, (const double*)d_fac, (const double*)d_wx,
+                           (const double*)d_sp, (const double*)d_B, mqf,
+                           (dgfs::cplx<T>*)pl->wtab);
+        return 0;
+    };
+    if (es == 8 ? tables(0.0) : tables(0.0f)) {
+        dgfs::set_error("bi_collision_plan_create: table kernels failed");
+        return fail(1);
     }
     if (hipGetLastError() != hipSuccess || hipDeviceSynchronize() != hipSuccess) {
         dgfs::set_error("bi_collision_plan_create: table kernels failed");
         return fail(1);
     }
-    for (void* p : {d_fac, d_wx, d_wc, d_sp, d_B, d_Bs}) (void)hipFree(p);
+    for (void* p : {d_fac, d_wx, d_wc, d_sp, d_B, d_Bs, d_yl}) (void)hipFree(p);
     *out = pl;
     return 0;
 }
@@ -267,10 +336,10 @@ extern "C" int dgfs_bi_collision_plan_query(dgfs_bi_collision_plan_t plan, int* 
                                               : dgfs::pick_split<float>(pl->N);
     if (chunk) *chunk = pl->chunk;
     if (scratch_bytes) {
-        const int S = pl->dtype == DGFS_F64 ? dgfs::pick_split<double>(pl->N)
-                                            : dgfs::pick_split<float>(pl->N);
-        const size_t acc = size_t(pl->Nrho) * pl->M * (S > 1 ? 2 : 1);
-        *scratch_bytes = (size_t(pl->chunk) * (4 + acc) + size_t(pl->ntask_max) * 2) * pl->n * cs;
+        const dgfs::BiSizes z = dgfs::bi_sizes_of(pl);
+        *scratch_bytes = (size_t(pl->chunk) * (4 * pl->n + z.Y + z.nyq + z.acc +
+                                               size_t(z.groups) * z.group) +
+                          size_t(pl->ntask_max) * 2 * pl->n) * cs;
     }
     return 0;
 }
@@ -280,11 +349,10 @@ extern "C" int dgfs_bi_collision_plan_destroy(dgfs_bi_collision_plan_t plan) {
     return 0;
 }
 
-extern "C" int dgfs_bi_collide(dgfs_bi_collision_plan_t plan, const void* up, const void* uq,
-                               void* Q, int K, int Ne, int ntask, const int* task_nterm,
-                               const int* task_slice, const void* task_coef, int ngroup,
-                               const int* group_start, const int* group_slice,
-                               hipStream_t stream) {
+static int bi_collide(dgfs_bi_collision_plan_t plan, const void* up, const void* uq, void* Q,
+                      int K, int Ne, int ntask, const int* task_nterm, const int* task_slice,
+                      const void* task_coef, int ngroup, const int* group_start,
+                      const int* group_slice, bool like, hipStream_t stream) {
     auto* pl = static_cast<BiPlan*>(plan);
     DGFS_REQUIRE(pl, "bi_collide: null plan");
     DGFS_REQUIRE(ntask >= 0 && ntask <= pl->ntask_max, "bi_collide: ntask=%d exceeds plan max %d",
@@ -296,9 +364,30 @@ extern "C" int dgfs_bi_collide(dgfs_bi_collision_plan_t plan, const void* up, co
                      group_slice,
                  "bi_collide: null pointer argument");
     dgfs::TaskView tv{K, Ne, int(pl->n), task_nterm, task_slice, task_coef};
-    if (pl->dtype == DGFS_F64)
-        return dgfs::bi_dispatch<double>(pl, up, uq, Q, tv, ntask, ngroup, group_start,
-                                         group_slice, stream);
-    return dgfs::bi_dispatch<float>(pl, up, uq, Q, tv, ntask, ngroup, group_start, group_slice,
-                                    stream);
+    auto run = [&](auto zero) {
+        using T = decltype(zero);
+        return dgfs::bi_for_grid<T>(pl->N, [&](auto g) {
+            return dgfs::bi_launch<T, int(g)>(pl, up, uq, Q, tv, ntask, ngroup, group_start,
+                                              group_slice, like, stream);
+        });
+    };
+    return pl->dtype == DGFS_F64 ? run(0.0) : run(0.0f);
+}
+
+extern "C" int dgfs_bi_collide(dgfs_bi_collision_plan_t plan, const void* up, const void* uq,
+                               void* Q, int K, int Ne, int ntask, const int* task_nterm,
+                               const int* task_slice, const void* task_coef, int ngroup,
+                               const int* group_start, const int* group_slice,
+                               hipStream_t stream) {
+    return bi_collide(plan, up, uq, Q, K, Ne, ntask, task_nterm, task_slice, task_coef, ngroup,
+                      group_start, group_slice, false, stream);
+}
+
+extern "C" int dgfs_bi_collide_like(dgfs_bi_collision_plan_t plan, const void* u, void* Q, int K,
+                                    int Ne, int ntask, const int* task_nterm,
+                                    const int* task_slice, const void* task_coef, int ngroup,
+                                    const int* group_start, const int* group_slice,
+                                    hipStream_t stream) {
+    return bi_collide(plan, u, u, Q, K, Ne, ntask, task_nterm, task_slice, task_coef, ngroup,
+                      group_start, group_slice, true, stream);
 }

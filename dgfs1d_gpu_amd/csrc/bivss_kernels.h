@@ -9,7 +9,7 @@
 //
 //   A  fwd   : F = FFT3(f_p)/n, G = FFT3(f_q)/n per task (the forward kernels
 //              of the single-species operator, collision_kernels.h)
-//   B  gain  : per (task, radius x, direction y, z-residue r):
+//   B  gain  : per (task, radius x, direction y):
 //                u1 = IFFT3(exp(+i m_q/(m_p+m_q) a_xy) F),
 //                u2 = IFFT3(exp(-i m_p/(m_p+m_q) a_xy) G)  (Fft3Engine, complex),
 //              and the forward transform along x of u1 u2 in registers
@@ -23,44 +23,47 @@
 //   D  line  : inverse along k1 and Q[out] += prefac (Re gain - f_p Re loss)
 //              (k_line_output of the single-species operator)
 //
-// Where the engine's LDS cube needs a residue split (FP64 N >= 24, FP32
-// N = 32), B is done by two streaming kernels instead (k_bi_yz: phase and the
-// l3, l2 inverses per l1 plane in LDS; k_bi_xprod: the l1 inverses, the
-// product and the forward x transform per pencil), so no work-group reloads F.
-//
-// Unlike the single-species operator the two inverse transforms are not
-// packed into one: with unequal mass fractions they carry different phases,
-// and both products are kept complex as in the reference.
+// This engine needs a product's whole cube in a work-group's LDS and keeps
+// both sides and the product complex.  Larger grids and larger task sets take
+// the streaming form of B to D (bi_pipeline.h).
 #pragma once
-#include "collision_kernels.h"
+#include "bi_pipeline.h"
+
+#include <algorithm>
 
 namespace dgfs {
 
 template <typename T, int N>
 constexpr int bi_split() { return pick_split<T>(N); }
 
-// grids whose gain cube needs a residue split take the two-kernel slab path
+// Which grids take the streaming kernels of bi_pipeline.h: all whose product
+// cube does not fit a work-group's LDS whole (FP64 N >= 24, FP32 N >= 32), and
+// N = 20 and FP32 N = 24 once a plan's products fill the chip.  Below that the
+// engine's fewer launches win, and at N <= 16 at every size that matters.
+// Microseconds for the four pairs, engine against streaming, M = 12, N_rho = 6
+// and 2, 8, 50 tasks: N = 16 FP32 160/205, 186/246, 503/526; N = 20 FP32
+// 223/293, 329/394, 1175/1008; N = 20 FP64 288/318, 603/531, 2499/1810; N = 24
+// FP32 253/283, 511/439, 2281/1438.
 template <typename T, int N>
-constexpr bool bi_slabs() { return bi_split<T, N>() > 1; }
+constexpr bool bi_engine() { return N <= 24 && bi_split<T, N>() == 1; }
+constexpr bool bi_streams(int N) { return N >= 20; }
+constexpr size_t kBiStreamBytes = size_t(48) << 20;    // of a plan's product cubes
 
-// B: one work-group per (task, xy, residue r).  acc layout
-// [t][xy][k1][r][y][j] with z = S*j + r (the layout k_bi_plane_part reads).
-template <typename T, int N, int S>
-__global__ void __launch_bounds__(round64(N * (N / S)))
+// B: one work-group per (task, xy); acc[t][xy][k1][y][z].
+template <typename T, int N>
+__global__ void __launch_bounds__(round64(N * N))
 k_bi_gain(const cplx<T>* __restrict__ Fhat, const cplx<T>* __restrict__ phase, int NXY,
           cplx<T>* __restrict__ acc_out) {
-    using E = Fft3Engine<T, N, S, round64(N * (N / S)), +1>;
-    constexpr int n = N * N * N, NS = N / S;
+    using E = Fft3Engine<T, N, 1, round64(N * N), +1>;
+    constexpr int n = N * N * N, NN = N * N;
     __shared__ cplx<T> V[E::LDS_ELEMS];
     const int lb = xcd_remap(blockIdx.x, gridDim.x);
-    const int r = lb % S;
-    const int xy = (lb / S) % NXY;
-    const int t = lb / (S * NXY);
+    const int xy = lb % NXY, t = lb / NXY;
     typename E::Split sp;
-    sp.init(r);
+    sp.init(0);
     const cplx<T>* ph = phase + size_t(xy) * 2 * 3 * N;     // [side][axis][l]
     auto map1 = [](int pp, int& i1, int& i2) { i1 = pp / N; i2 = pp - (pp / N) * N; };
-    auto map3 = [](int P, int& o2, int& j) { o2 = P / NS; j = P - (P / NS) * NS; };
+    auto map3 = [](int P, int& o2, int& j) { o2 = P / N; j = P - (P / N) * N; };
     cplx<T> R1[N];
     sfor<0, 2>([&](auto Si) {
         constexpr int side = Si;
@@ -68,7 +71,7 @@ k_bi_gain(const cplx<T>* __restrict__ Fhat, const cplx<T>* __restrict__ phase, i
         const cplx<T>* e = ph + side * 3 * N;
         // the separable phase exp(i th_1 l1) exp(i th_2 l2) exp(i th_3 l3) is
         // applied per axis just before that axis' transform: l3 in the load,
-        // l2 in pass 2 and l1 in pass 3 (these touch only this residue's data)
+        // l2 in pass 2 and l1 in pass 3
         E::run(V, sp, map1,
                [&](int i1, int i2, int i3) { return e[2 * N + i3] * F[(size_t(i3) * N + i1) * N + i2]; },
                [&](auto I, cplx<T> v) { return e[N + int(I)] * v; }, map3,
@@ -82,89 +85,21 @@ k_bi_gain(const cplx<T>* __restrict__ Fhat, const cplx<T>* __restrict__ phase, i
                        RegDFT<T, N, -1>::template run<1, 0>(pr, R1);
                        cplx<T>* dst = acc_out + (size_t(t) * NXY + xy) * n;
                        sfor<0, N>([&](auto I) {
-                           dst[((size_t(I) * S + r) * N + o2) * NS + j] = R1[I];
+                           dst[size_t(I) * NN + o2 * N + j] = R1[I];
                        });
                    }
                });
     });
 }
 
-// B', for grids whose engine cube does not fit LDS whole (residue split
-// S > 1): two streaming kernels instead of k_bi_gain, so that no work-group
-// reloads F.
-// B'1: one N-thread slot per plane (t, xy, side, l1): P[l2][l3] =
-//      e1(l1) e2(l2) e3(l3) F[l3][l1][l2], inverse along l3 then l2 in LDS ->
-//      Y[t][xy][side][l1][y][z].
-template <typename T, int N>
-__global__ void __launch_bounds__(planes_per_wg(N) * N)
-k_bi_yz(const cplx<T>* __restrict__ Fhat, const cplx<T>* __restrict__ phase, int NXY,
-        long nplanes, cplx<T>* __restrict__ Y) {
-    constexpr int PL = planes_per_wg(N), NT = PL * N, NN = N * N, n = N * NN, PS = N * (N + 1);
-    __shared__ cplx<T> L[PL * PS];
-    const long plane0 = long(blockIdx.x) * PL;
-    const int pl = threadIdx.x / N, c = threadIdx.x - pl * N;
-    const long pid = plane0 + pl;
-    const bool live = pid < nplanes;
-    cplx<T>* P = L + pl * PS;
-    if (live) {
-        const int l1 = int(pid % N);
-        const long tws = pid / N;                      // (t*NXY + xy)*2 + side
-        const int side = int(tws % 2);
-        const long txy = tws / 2;
-        const int xy = int(txy % NXY);
-        const long t = txy / NXY;
-        const cplx<T>* F = Fhat + (size_t(t) * 2 + side) * n + size_t(l1) * N + c;
-        const cplx<T>* e = phase + (size_t(xy) * 2 + side) * 3 * N;
-        const cplx<T> e12 = e[l1] * e[N + c];          // thread c = l2
-        sfor<0, N>([&](auto J) {
-            P[c * (N + 1) + J] = (e12 * e[2 * N + J]) * F[size_t(J) * NN];
-        });
-    }
-    __syncthreads();
-    if (live) lds_fft_row<T, N, +1>(P, c);     // row l2: l3 -> z
-    __syncthreads();
-    if (live) lds_fft_col<T, N, +1>(P, c);     // column z: l2 -> y
-    __syncthreads();
-    for (int k = threadIdx.x; k < PL * NN; k += NT) {
-        const int q = k / NN, r = k - q * NN;
-        const long pq = plane0 + q;
-        if (pq >= nplanes) continue;
-        Y[pq * NN + r] = L[q * PS + (r / N) * (N + 1) + r % N];     // [y][z]
-    }
-}
-
-// B'2: one thread per (t, xy, y, z) pencil: u1, u2 = inverse along l1 of the
-// two sides, forward along x of u1 u2, written over side 0's pencil
-// (acc[t][xy][k1][y][z] with stride 2n per (t, xy)).
-template <typename T, int N>
-__global__ void __launch_bounds__(256)
-k_bi_xprod(long npen, cplx<T>* __restrict__ Y) {
-    constexpr int NN = N * N, n = N * NN;
-    const long gid = long(blockIdx.x) * 256 + threadIdx.x;
-    if (gid >= npen) return;
-    const long txy = gid / NN;
-    const int yz = int(gid - txy * NN);
-    cplx<T>* Y0 = Y + txy * 2 * n + yz;
-    const cplx<T>* Y1 = Y0 + n;
-    cplx<T> a[N], R1[N], o[N];
-    sfor<0, N>([&](auto I) { a[I] = Y0[size_t(I) * NN]; });
-    RegDFT<T, N, +1>::template run<1, 0>(a, R1);
-    sfor<0, N>([&](auto I) { a[I] = Y1[size_t(I) * NN]; });
-    RegDFT<T, N, +1>::template run<1, 0>(a, o);
-    sfor<0, N>([&](auto I) { a[I] = R1[I] * o[I]; });
-    RegDFT<T, N, -1>::template run<1, 0>(a, R1);
-    sfor<0, N>([&](auto I) { Y0[size_t(I) * NN] = R1[I]; });
-}
-
 // C1: one work-group per (t, k1, xy-group g): slot s of PL takes the group's
 // xy = xy0 + s, xy0 + s + PL, ...; the group's partial
 // G^_g(k1, :, :) = sum_xy W_xy FFT2_{y,z}(acc_xy(k1)) goes to
-// Gp[t][g][k1][k2][k3].  acc of (t, xy) starts at (t*NXY + xy)*accstride.
+// Gp[t][g][k1][k2][k3].
 template <typename T, int N>
 __global__ void __launch_bounds__(planes_per_wg(N) * N)
-k_bi_plane_part(const cplx<T>* __restrict__ acc_in, long accstride,
-                const cplx<T>* __restrict__ wtab, int NXY, int SB, int XG,
-                cplx<T>* __restrict__ Gp) {
+k_bi_plane_part(const cplx<T>* __restrict__ acc_in, const cplx<T>* __restrict__ wtab, int NXY,
+                int XG, cplx<T>* __restrict__ Gp) {
     constexpr int PL = planes_per_wg(N), NN = N * N, n = N * NN, PS = N * (N + 1);
     __shared__ cplx<T> L[PL * PS];
     const int g = blockIdx.x % XG;
@@ -174,7 +109,6 @@ k_bi_plane_part(const cplx<T>* __restrict__ acc_in, long accstride,
     const int per = (NXY + XG - 1) / XG;
     const int xy0 = g * per < NXY ? g * per : NXY;
     const int xy1 = xy0 + per < NXY ? xy0 + per : NXY;
-    const int NSB = N / SB;
     cplx<T> G[N];
     sfor<0, N>([&](auto I) { G[I] = mk(T(0), T(0)); });
     const int nround = (xy1 - xy0 + PL - 1) / PL;
@@ -183,12 +117,8 @@ k_bi_plane_part(const cplx<T>* __restrict__ acc_in, long accstride,
         const bool live = xy < xy1;
         __syncthreads();
         if (live) {
-            const cplx<T>* src = acc_in + (size_t(t) * NXY + xy) * accstride + size_t(k1) * NN;
-            for (int pos = c; pos < NN; pos += N) {
-                const int r = pos / (N * NSB), rem = pos - r * N * NSB;
-                const int y = rem / NSB, z = (rem - y * NSB) * SB + r;
-                P[y * (N + 1) + z] = src[pos];
-            }
+            const cplx<T>* src = acc_in + (size_t(t) * NXY + xy) * n + size_t(k1) * NN;
+            for (int y = 0; y < N; ++y) P[y * (N + 1) + c] = src[y * N + c];
         }
         __syncthreads();
         if (live) lds_fft_row<T, N, -1>(P, c);     // z -> k3
@@ -268,84 +198,175 @@ struct BiPlan {
     int N, M, Nrho, Mpre, dtype, ntask_max, chunk;
     double prefac, mp, mq;
     size_t n;
-    void* phase = nullptr;  // [Nrho*M][2][3][N] cplx<T>
-    void* wtab = nullptr;   // [Nrho*M][k1][k2][k3] cplx<T>  qw sw / n * b_pq
-    void* ctab = nullptr;   // [l1][l2][l3] cplx<T>  c_pq
+    bool stream = false;    // the streaming kernels (bi_pipeline.h)
+    bool antipodal = false; // the streaming form's products come in opposite pairs (2u, 2u + 1)
+    int xg_max = 1;         // groups of k_bi_sum that Gp holds
+    void* phase = nullptr;  // [Nrho*M][2][3][N] cplx<T>, in product order
+    void* wtab = nullptr;   // [Nrho*M][k1][k2][k3] cplx<T>  qw sw / n * b_pq; streaming: k_bi_wtab
+    void* wspec = nullptr;  // streaming: the weights at k1 = N/2 (k_bi_wtab)
+    void* ctab = nullptr;   // [l1][l2][l3] cplx<T>  c_pq; streaming: k_bi_chtab
     void* Fhat = nullptr;   // [chunk][2][n] cplx<T>
     void* Iw = nullptr;     // [chunk][2][n] cplx<T>
-    void* acc = nullptr;    // [chunk][Nrho*M][n] cplx<T>, or [chunk][Nrho*M][2][n] on the slab path
-    void* H = nullptr;      // [ntask_max][2][n] cplx<T>
-    void* Gp = nullptr;     // [chunk][xgroups_max][n] cplx<T>  partial G^ per xy group
+    void* Y = nullptr;      // streaming: [chunk][Nrho*M][n] cplx<T>
+    void* nyq = nullptr;    // streaming: [chunk][Nrho*M][3][N*N] cplx<T>
+    void* acc = nullptr;    // [chunk][Nrho*M][n] cplx<T>; streaming: [chunk][Nrho*M][N + XS][NPT]
+    void* H = nullptr;      // [ntask_max][2][n] cplx<T>: loss, gain
+    void* norm = nullptr;   // streaming: [chunk][2][bi_norm_blocks] FP64
+    void* Gp = nullptr;     // [chunk][groups][n] cplx<T>  partial G^; streaming: [..][H][NPT][2]
 };
 
+// The streaming form for nt tasks: forward plane transforms of f, g in Iw ->
+// the x-planes of loss and gain in Z.  The groups and ranges spread a small task set over the chip:
+// each kernel gets at least the 2048 waves that are resident at two per SIMD
+// where the task set allows it (finer groups reload F and G, more ranges add
+// their k1 = N/2 planes: twice the waves made the 6-task N = 24 set 8 % slower).
+template <typename T, int N>
+int bi_stream_chunk(BiPlan* pl, int nt, bool like, cplx<T>* Z, hipStream_t st) {
+    using Gm = BiGeo<N>;
+    using Pl = BiPlane<T, N>;
+    const int dstride = like ? 2 : 1;
+    const int ND = pl->Nrho * pl->M / dstride;
+    const int NU = pl->antipodal ? pl->Nrho * pl->M / 2 : ND;
+    const cplx<T>* F = (const cplx<T>*)pl->Fhat;
+    const cplx<T>* ph = (const cplx<T>*)pl->phase;
+    double* norm = (double*)pl->norm;
+    hipLaunchKernelGGL((k_bi_fwd_line<T, N>), dim3(nt * 2 * bi_norm_blocks(N)), dim3(256), 0, st,
+                       (const cplx<T>*)pl->Iw, (cplx<T>*)pl->Fhat, norm);
+    DGFS_HIP_CHECK(hipGetLastError());
+    auto groups = [](long want, long have, int most) {
+        const long g = (want + have - 1) / have;
+        return int(g < 1 ? 1 : (g > most ? most : g));
+    };
+    const int PB = (Gm::NN + kBiXWG / 2 - 1) / (kBiXWG / 2);
+    const int XGX = groups(2048, long(nt) * PB * (kBiXWG / 64), (ND + 1) / 2);
+    const int nxb = nt * PB * XGX;
+    const long nny = long(nt) * ND * 3;
+    constexpr int NPW = BiNyq<T, N>::PW;
+    hipLaunchKernelGGL((k_bi_x<T, N>), dim3(nxb + (nny + NPW - 1) / NPW), dim3(kBiXWG), 0, st, F, ph,
+                       norm, ND, dstride, PB, XGX, nxb, (cplx<T>*)pl->Y, nny, (cplx<T>*)pl->nyq);
+    DGFS_HIP_CHECK(hipGetLastError());
+    int XS = 1;
+    for (int d = 2; d <= kBiXSMax; ++d)
+        if (N % d == 0 && long(nt) * ND * XS * Pl::PT / 64 < 2048) XS = d;
+    const long ns = long(nt) * ND * XS;
+    hipLaunchKernelGGL((k_bi_plane<T, N>), dim3((ns + Pl::PW - 1) / Pl::PW), dim3(Pl::WG), 0, st,
+                       (const cplx<T>*)pl->Y, (const cplx<T>*)pl->nyq, ns, XS, (cplx<T>*)pl->acc);
+    DGFS_HIP_CHECK(hipGetLastError());
+    const int QB = (Gm::NPT + kBiSumWG / 2 - 1) / (kBiSumWG / 2);
+    // whole units per group; Gp holds chunk * xg_max groups
+    int XG = groups(2048, long(nt) * QB * (kBiSumWG / 64), NU);
+    XG = int(std::min<long>(XG, long(pl->xg_max) * pl->chunk / nt));
+    XG = (NU + (NU + XG - 1) / XG - 1) / ((NU + XG - 1) / XG);
+    auto* sum = like ? k_bi_sum<T, N, kBiReal>
+                     : (pl->antipodal ? k_bi_sum<T, N, kBiPair> : k_bi_sum<T, N, kBiComplex>);
+    hipLaunchKernelGGL(sum, dim3(nt * QB * XG), dim3(kBiSumWG), 0, st, (const cplx<T>*)pl->acc,
+                       (const cplx<T>*)pl->wtab, (const cplx<T>*)pl->wspec, nt, ND, XS, NU, XG, QB,
+                       (cplx<T>*)pl->Gp);
+    DGFS_HIP_CHECK(hipGetLastError());
+    const int QF = (Gm::NPH + 31) / 32;
+    hipLaunchKernelGGL((k_bi_pen<T, N>), dim3(nt * QF), dim3(kBiPenWG), 0, st, (const cplx<T>*)pl->Gp,
+                       XG, QF, F, norm, (const cplx<T>*)pl->ctab, Z);
+    DGFS_HIP_CHECK(hipGetLastError());
+    return 0;
+}
+
+// like: up = uq and every task's f and g terms are the same
 template <typename T, int N>
 int bi_launch(BiPlan* pl, const void* up, const void* uq, void* Q, TaskView tv, int ntask,
-              int ngroup, const int* gstart, const int* gslice, hipStream_t st) {
-    constexpr int S = bi_split<T, N>();
-    constexpr int PL = planes_per_wg(N);
+              int ngroup, const int* gstart, const int* gslice, bool like, hipStream_t st) {
     constexpr long NN = long(N) * N;
     const int NXY = pl->Nrho * pl->M;
     const size_t n = pl->n;
+    like = like && pl->antipodal && pl->mp == pl->mq;
     for (int c0 = 0; c0 < ntask; c0 += pl->chunk) {
         const int nt = ntask - c0 < pl->chunk ? ntask - c0 : pl->chunk;
         TaskView tc = tv;
         tc.nterm = tv.nterm + 2 * size_t(c0);
         tc.slice = tv.slice + size_t(c0) * 2 * tv.K;
         tc.coef = static_cast<const T*>(tv.coef) + size_t(c0) * 2 * tv.K;
-        const int XG = bi_xgroups<N>(nt, NXY);
         const long npl = long(nt) * 2 * N;
         constexpr int FP = fwd_planes_per_wg(N);
         hipLaunchKernelGGL((k_fwd_plane<T, N, false>), dim3((npl + FP - 1) / FP), dim3(FP * N),
                            0, st, (const T*)up, (const T*)uq, tc, 2, npl, (cplx<T>*)pl->Iw);
         DGFS_HIP_CHECK(hipGetLastError());
-        const long nli = long(nt) * 2 * NN;
-        hipLaunchKernelGGL((k_fwd_line<T, N>), dim3((nli + 255) / 256), dim3(256), 0, st, nli, 2,
-                           (const cplx<T>*)pl->Iw, (cplx<T>*)pl->Fhat);
-        DGFS_HIP_CHECK(hipGetLastError());
-        if constexpr (bi_slabs<T, N>()) {
-            const long npl2 = long(nt) * NXY * 2 * N;
-            hipLaunchKernelGGL((k_bi_yz<T, N>), dim3((npl2 + PL - 1) / PL), dim3(PL * N), 0, st,
-                               (const cplx<T>*)pl->Fhat, (const cplx<T>*)pl->phase, NXY, npl2,
+        bool done = false;
+        if constexpr (bi_streams(N)) if (pl->stream) {
+            if (int rc = bi_stream_chunk<T, N>(pl, nt, like, (cplx<T>*)pl->H + size_t(c0) * 2 * n,
+                                               st))
+                return rc;
+            done = true;
+        }
+        if constexpr (bi_engine<T, N>()) if (!done) {
+            constexpr int PL = planes_per_wg(N);
+            const int XG = bi_xgroups<N>(nt, NXY);
+            const long nli = long(nt) * 2 * NN;
+            hipLaunchKernelGGL((k_fwd_line<T, N>), dim3((nli + 255) / 256), dim3(256), 0, st, nli,
+                               2, (const cplx<T>*)pl->Iw, (cplx<T>*)pl->Fhat);
+            DGFS_HIP_CHECK(hipGetLastError());
+            hipLaunchKernelGGL((k_bi_gain<T, N>), dim3(nt * NXY), dim3(round64(N * N)), 0, st,
+                               (const cplx<T>*)pl->Fhat, (const cplx<T>*)pl->phase, NXY,
                                (cplx<T>*)pl->acc);
             DGFS_HIP_CHECK(hipGetLastError());
-            const long npen = long(nt) * NXY * NN;
-            hipLaunchKernelGGL((k_bi_xprod<T, N>), dim3((npen + 255) / 256), dim3(256), 0, st,
-                               npen, (cplx<T>*)pl->acc);
-            DGFS_HIP_CHECK(hipGetLastError());
             hipLaunchKernelGGL((k_bi_plane_part<T, N>), dim3(nt * N * XG), dim3(PL * N), 0, st,
-                               (const cplx<T>*)pl->acc, long(2 * n), (const cplx<T>*)pl->wtab,
-                               NXY, 1, XG, (cplx<T>*)pl->Gp);
+                               (const cplx<T>*)pl->acc, (const cplx<T>*)pl->wtab, NXY, XG,
+                               (cplx<T>*)pl->Gp);
             DGFS_HIP_CHECK(hipGetLastError());
-        } else {
-            hipLaunchKernelGGL((k_bi_gain<T, N, S>), dim3(nt * NXY * S),
-                               dim3(round64(N * (N / S))), 0, st, (const cplx<T>*)pl->Fhat,
-                               (const cplx<T>*)pl->phase, NXY, (cplx<T>*)pl->acc);
-            DGFS_HIP_CHECK(hipGetLastError());
-            hipLaunchKernelGGL((k_bi_plane_part<T, N>), dim3(nt * N * XG), dim3(PL * N), 0, st,
-                               (const cplx<T>*)pl->acc, long(n), (const cplx<T>*)pl->wtab, NXY,
-                               S, XG, (cplx<T>*)pl->Gp);
+            hipLaunchKernelGGL((k_bi_plane_fin<T, N>), dim3(nt * N), dim3(PL * N), 0, st,
+                               (const cplx<T>*)pl->Gp, XG, (const cplx<T>*)pl->Fhat,
+                               (const cplx<T>*)pl->ctab, (cplx<T>*)pl->H + size_t(c0) * 2 * n);
             DGFS_HIP_CHECK(hipGetLastError());
         }
-        hipLaunchKernelGGL((k_bi_plane_fin<T, N>), dim3(nt * N), dim3(PL * N), 0, st,
-                           (const cplx<T>*)pl->Gp, XG, (const cplx<T>*)pl->Fhat,
-                           (const cplx<T>*)pl->ctab, (cplx<T>*)pl->H + size_t(c0) * 2 * n);
+    }
+    if constexpr (bi_streams(N)) if (pl->stream) {
+        using Pl = BiPlane<T, N>;
+        const long ns = long(ngroup) * N;
+        hipLaunchKernelGGL((k_bi_out<T, N>), dim3((ns + Pl::PW - 1) / Pl::PW), dim3(Pl::WG), 0, st,
+                           (const T*)up, tv, (const cplx<T>*)pl->H, ns, gstart, gslice,
+                           T(pl->prefac), (T*)Q);
+        DGFS_HIP_CHECK(hipGetLastError());
+        return 0;
+    }
+    if constexpr (bi_engine<T, N>()) {
+        const long nlo = long(ngroup) * NN;
+        hipLaunchKernelGGL((k_line_output<T, N, false>),
+                           dim3((nlo * line_lanes(N) + kLineWG - 1) / kLineWG), dim3(kLineWG), 0,
+                           st, (const T*)up, (const T*)nullptr, (const double*)nullptr, tv,
+                           (const cplx<T>*)pl->H, nlo, gstart, gslice, T(pl->prefac), (T*)Q);
         DGFS_HIP_CHECK(hipGetLastError());
     }
-    const long nlo = long(ngroup) * NN;
-    hipLaunchKernelGGL((k_line_output<T, N, false>),
-                       dim3((nlo * line_lanes(N) + kLineWG - 1) / kLineWG), dim3(kLineWG), 0, st,
-                       (const T*)up, (const T*)nullptr, (const double*)nullptr, tv,
-                       (const cplx<T>*)pl->H, nlo, gstart, gslice, T(pl->prefac), (T*)Q);
-    DGFS_HIP_CHECK(hipGetLastError());
     return 0;
 }
 
-#define DGFS_BI_EXTERN(T, N)                                                              \
-    extern template int bi_launch<T, N>(BiPlan*, const void*, const void*, void*, TaskView, \
-                                        int, int, const int*, const int*, hipStream_t);
-#define DGFS_BI_INST(T, N)                                                                \
+// the streaming form's weight tables (FP64 device inputs, see k_bi_wtab)
+template <typename T, int N>
+int bi_stream_tables(BiPlan* pl, const int* ylist, const double* fac, const double* wx,
+                     const double* szpre, const double* Bt, const double* wc, const double* Bsum,
+                     double mqf) {
+    if constexpr (!bi_streams(N)) return 1;
+    using Gm = BiGeo<N>;
+    hipLaunchKernelGGL((k_bi_chtab<T, N>), dim3((N * Gm::NPH + 31) / 32), dim3(256), 0, 0,
+                       pl->Nrho, pl->Mpre, fac, wc, szpre, Bsum, (cplx<T>*)pl->ctab);
+    const int us = pl->antipodal ? 2 : 1, NU = pl->Nrho * pl->M / us;
+    const long per = long(N) * Gm::NPT + Gm::NPH;
+    hipLaunchKernelGGL((k_bi_wtab<T, N>), dim3((NU * per + 255) / 256), dim3(256), 0, 0, pl->M, NU,
+                       us, pl->Mpre, ylist, fac, wx, szpre, Bt, mqf, (cplx<T>*)pl->wtab,
+                       (cplx<T>*)pl->wspec);
+    return hipGetLastError() == hipSuccess ? 0 : 1;
+}
+
+#define DGFS_BI_SIG(T, N)                                                                  \
     template int bi_launch<T, N>(BiPlan*, const void*, const void*, void*, TaskView, int, int, \
-                                 const int*, const int*, hipStream_t);
+                                 const int*, const int*, bool, hipStream_t);               \
+    template int bi_stream_tables<T, N>(BiPlan*, const int*, const double*, const double*, \
+                                        const double*, const double*, const double*, \
+                                        const double*, double);
+#define DGFS_BI_EXTERN(T, N)                                                               \
+    extern template int bi_launch<T, N>(BiPlan*, const void*, const void*, void*, TaskView, int, \
+                                        int, const int*, const int*, bool, hipStream_t);   \
+    extern template int bi_stream_tables<T, N>(BiPlan*, const int*, const double*, const double*, \
+                                               const double*, const double*, const double*, \
+                                               const double*, double);
+#define DGFS_BI_INST(T, N) DGFS_BI_SIG(T, N)
 
 DGFS_COLLIDE_SIZES(DGFS_BI_EXTERN, float)
 DGFS_BI_EXTERN(float, 48)

@@ -149,7 +149,7 @@ int dgfs_collision_timing_read(dgfs_collision_plan_t plan, double* ms /*[5]*/, i
  *   szpre    Mpre x 3 full-sphere pre-rule (scattering.py:55-61), swpre = 4 pi / Mpre
  *   mp, mq   masses of the species pair (molar mass / molarMass0)
  *   alpha, omega  VSS parameters of the pair; prefac as scattering.py:86-90
- * Tasks are processed in chunks whose gain products fit a 2 GiB scratch
+ * Tasks are processed in chunks whose gain products fit a 4 GiB scratch
  * (environment variable DGFS_BI_SCRATCH_MB, read at plan creation, sets
  * another budget; at least one task per chunk). */
 typedef void* dgfs_bi_collision_plan_t;
@@ -172,6 +172,14 @@ int dgfs_bi_collide(dgfs_bi_collision_plan_t plan, const void* up, const void* u
                     int K, int Ne, int ntask, const int* task_nterm, const int* task_slice,
                     const void* task_coef, int ngroup, const int* group_start,
                     const int* group_slice, hipStream_t stream);
+/* dgfs_bi_collide(plan, u, u, Q, ...) for task tables whose f and g terms are
+ * the same in every task (a species with itself on a nodal basis).  With
+ * equal masses and antipodally symmetric rules opposite directions share one
+ * product, which halves the work; otherwise the same as dgfs_bi_collide. */
+int dgfs_bi_collide_like(dgfs_bi_collision_plan_t plan, const void* u, void* Q, int K, int Ne,
+                         int ntask, const int* task_nterm, const int* task_slice,
+                         const void* task_coef, int ngroup, const int* group_start,
+                         const int* group_slice, hipStream_t stream);
 
 /* Linear minmod slope limiter (reference limitLin,
  * dgfs1D/astd/kernels/limiters.mako:17-76, applied by astd/abstd.py:402-416

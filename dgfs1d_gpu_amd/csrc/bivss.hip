@@ -149,7 +149,7 @@ static std::vector<int> opposite(const double* p, int n) {
 
 // scratch budget of the gain products: tasks are processed in chunks whose
 // [chunk][Nrho*M][n] complex products fit in it
-constexpr size_t kBiAccBudget = size_t(4) << 30;
+constexpr size_t kBiAccBudget = size_t(8) << 30;
 
 }  // namespace dgfs
 

@@ -301,7 +301,7 @@ int bi_launch(BiPlan* pl, const void* up, const void* uq, void* Q, TaskView tv, 
             const int XG = bi_xgroups<N>(nt, NXY);
             const long nli = long(nt) * 2 * NN;
             hipLaunchKernelGGL((k_fwd_line<T, N>), dim3((nli + 255) / 256), dim3(256), 0, st, nli,
-                               2, (const cplx<T>*)pl->Iw, (cplx<T>*)pl->Fhat);
+                               2, (const cplx<T>*)pl->Iw, (cplx<T>*)pl->Fhat, (cplx<T>*)nullptr);
             DGFS_HIP_CHECK(hipGetLastError());
             hipLaunchKernelGGL((k_bi_gain<T, N>), dim3(nt * NXY), dim3(round64(N * N)), 0, st,
                                (const cplx<T>*)pl->Fhat, (const cplx<T>*)pl->phase, NXY,

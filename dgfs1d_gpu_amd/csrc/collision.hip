@@ -182,9 +182,10 @@ extern "C" int dgfs_collision_plan_create(int N, int M, int Nrho, double L, cons
     pl->QG_cap = pl->QG;
     hipError_t e3 = hipMalloc(&pl->Iw, size_t(ntask_max) * 2 * n * cs);
     hipError_t e4 = hipMalloc(&pl->H, size_t(ntask_max) * 3 * n * cs);   // 3 planes: reference-state form
+    hipError_t e6 = hipMalloc(&pl->FN, size_t(ntask_max) * 2 * 3 * N * N * cs);
     hipError_t e5 = hipMalloc(&pl->nyq, size_t(ntask_max) * 2 * Nrho * M * 6 * N * N * es);
     if (e1 != hipSuccess || e2 != hipSuccess || e3 != hipSuccess || e4 != hipSuccess ||
-        e5 != hipSuccess) {
+        e5 != hipSuccess || e6 != hipSuccess) {
         dgfs::set_error("collision_plan_create: scratch allocation failed");
         dgfs_collision_plan_destroy(pl);
         return 1;
@@ -237,7 +238,7 @@ extern "C" int dgfs_collision_plan_destroy(dgfs_collision_plan_t plan) {
     auto* pl = static_cast<CollisionPlan*>(plan);
     if (!pl) return 0;
     free_events(pl);
-    for (void* p : {pl->phase, pl->phz, pl->wtab, pl->bb2, pl->Fhat, pl->acc, pl->Iw, pl->H, pl->nyq,
+    for (void* p : {pl->phase, pl->phz, pl->wtab, pl->bb2, pl->Fhat, pl->acc, pl->Iw, pl->H, pl->FN, pl->nyq,
                     pl->Fhat0, pl->ucache})
         if (p) (void)hipFree(p);
     delete pl;

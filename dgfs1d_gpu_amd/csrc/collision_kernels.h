@@ -155,11 +155,17 @@ k_fwd_plane(const T* __restrict__ u, const T* __restrict__ ug, TaskView tv, int 
     }
 }
 
+// order of an element (row r, column c) of a Nyquist plane in k_nyq's lanes
+template <int N>
+DGFS_DEV int nyq_at(int r, int c) { return (c >> 1) * 2 * N + 2 * r + (c & 1); }
+
 // A2: line (l3, l2) of task-which tw: transform over x, scale 1/n;
-//     F^[t][which][l3][l1][l2]
+//     F^[t][which][l3][l1][l2], and the three Nyquist planes of F^ once more
+//     as k_nyq reads them, FN[t][which][3][nyq_at] (FN null: not wanted)
 template <typename T, int N>
 __global__ void __launch_bounds__(256)
-k_fwd_line(long nlines, int nfg, const cplx<T>* __restrict__ Iw, cplx<T>* __restrict__ Fhat) {
+k_fwd_line(long nlines, int nfg, const cplx<T>* __restrict__ Iw, cplx<T>* __restrict__ Fhat,
+           cplx<T>* __restrict__ FN) {
     constexpr int NN = N * N;
     const long gid = long(blockIdx.x) * 256 + threadIdx.x;
     if (gid >= nlines) return;
@@ -173,7 +179,16 @@ k_fwd_line(long nlines, int nfg, const cplx<T>* __restrict__ Iw, cplx<T>* __rest
     const T inv_n = T(1) / T(N * NN);
     const int l3 = r / N, l2 = r - l3 * N;
     cplx<T>* dst = Fhat + (size_t(t) * 2 + which) * size_t(N) * NN + size_t(l3) * NN + l2;
-    sfor<0, N>([&](auto K1) { dst[size_t(K1) * N] = inv_n * o[K1]; });
+    sfor<0, N>([&](auto K1) {
+        o[K1] = inv_n * o[K1];
+        dst[size_t(K1) * N] = o[K1];
+    });
+    if (FN == nullptr) return;
+    constexpr int H = N / 2;
+    cplx<T>* fn = FN + (size_t(t) * 2 + which) * 3 * NN;
+    fn[nyq_at<N>(l2, l3)] = o[H];                                     // l1 = N/2: (l2, l3)
+    if (l2 == H) sfor<0, N>([&](auto K1) { fn[NN + nyq_at<N>(l3, K1)] = o[K1]; });
+    if (l3 == H) sfor<0, N>([&](auto K1) { fn[2 * NN + nyq_at<N>(l2, K1)] = o[K1]; });
 }
 
 // ================================================================ kernel B
@@ -192,60 +207,55 @@ k_fwd_line(long nlines, int nfg, const cplx<T>* __restrict__ Iw, cplx<T>* __rest
 //   C: l3 = N/2, l1, l2 != N/2  -> (-1)^z C(x, y)
 // k_nyq writes Im of A+-, B+-, C+- for every (task, which, p, q):
 // nyq[t][w][p][q][6][N*N] with planes A+ A- [y][z], B+ B- [z][x], C+ C- [y][x].
+// beta and delta of one plane are real fields, so one complex transform
+// carries both: beta + i delta has the spectrum (kap - i conj kap) F^ with
+// kap = (e - e~)/(2i), e~ the phase with the conjugate factor on every Nyquist
+// axis (the spectrum of Im IFFT3(e F^)), and kap - i conj kap =
+// (1 - i)(Re kap - Im kap): three transforms per (p, q) on lane pairs.  The
+// planes of F^ come gathered (FN): two of them are strided in F^, one line of
+// memory per element, and those reads bound the kernel (six planes of
+// e^{+-ia} F^ on single lanes took the same 240 us for 96 tasks x 192 (p, q),
+// N = 32, FP32, as these three did from F^; from FN they take 178 us).  Bound
+// by its stores.
 template <typename T, int N>
 __global__ void __launch_bounds__(6 * N)
-k_nyq(const cplx<T>* __restrict__ Fhat, const cplx<T>* __restrict__ phase, int M, int Nrho,
+k_nyq(const cplx<T>* __restrict__ FN, const cplx<T>* __restrict__ phase, int M, int Nrho,
       int NW, T* __restrict__ nyq) {
-    // one 2D plane per N-thread slot: slot = 2 type + sign; thread c walks k
-    constexpr int NN = N * N, n = N * NN, PS = N * (N + 1), H = N / 2;
-    __shared__ cplx<T> L[6 * PS];
+    // slot s of 2N threads takes one plane; rows a and columns b by slot:
+    // A: (l2, l3), B: (l3, l1), C: (l2, l1)
+    constexpr int NN = N * N, H = N / 2, PI = N + 1;
+    __shared__ cplx<T> L[3 * N * PI];
     const int bid = blockIdx.x;
     const int q = bid % M, p = (bid / M) % Nrho, w = (bid / (M * Nrho)) % NW;
     const int t = bid / (M * Nrho * NW);
-    const cplx<T>* F = Fhat + (size_t(t) * 2 + w) * n;
     const cplx<T>* ph = phase + (size_t(p) * M + q) * 3 * N;
-    const int slot = threadIdx.x / N, c = threadIdx.x - slot * N;
-    const int type = slot >> 1;
-    const bool minus = (slot & 1) != 0;
-    cplx<T>* P = L + slot * PS;
-    // loads: rows a, columns b of the plane (A: a = l2, b = l3; B: a = l1,
-    // b = l3; C: a = l1, b = l2); consecutive threads read consecutive l2
-    // where the plane has an l2 axis (A, C)
-    if (type == 0) {                       // thread c = l2, k = l3
-        const cplx<T> e0 = ph[H] * ph[N + c];
-        sfor<0, N>([&](auto K) {
-            constexpr int k = K;
-            const cplx<T> e = e0 * ph[2 * N + k];
-            P[c * (N + 1) + k] = cmul_conj_if(F[(size_t(k) * N + H) * N + c], e, minus);
-        });
-    } else if (type == 1) {                // thread c = l1, k = l3
-        const cplx<T> e0 = ph[c] * ph[N + H];
-        const bool zero = c == H;
-        sfor<0, N>([&](auto K) {
-            constexpr int k = K;
-            const cplx<T> e = e0 * ph[2 * N + k];
-            const cplx<T> v = cmul_conj_if(F[(size_t(k) * N + c) * N + H], e, minus);
-            P[c * (N + 1) + k] = zero ? mk(T(0), T(0)) : v;
-        });
-    } else {                               // thread c = l2, k = l1
-        const cplx<T> e0 = ph[N + c] * ph[2 * N + H];
-        sfor<0, N>([&](auto K) {
-            constexpr int k = K;
-            const cplx<T> e = ph[k] * e0;
-            const cplx<T> v = cmul_conj_if(F[(size_t(H) * N + k) * N + c], e, minus);
-            P[k * (N + 1) + c] = (k == H || c == H) ? mk(T(0), T(0)) : v;
-        });
-    }
+    const int s = threadIdx.x / (2 * N), u = threadIdx.x - s * 2 * N, r = u >> 1, h = u & 1;
+    const cplx<T>* F = FN + ((size_t(t) * 2 + w) * 3 + s) * NN + u;
+    const int ra = s == 1 ? 2 : 1, ca = s == 0 ? 2 : 0;              // row, column axes; s is fixed
+    const cplx<T> E = ph[s * N + H], er = ph[ra * N + r];
+    const cplx<T> erE = E * er, ert = conj(E) * (r == H ? conj(er) : er);
+    // B leaves l1 = N/2 to A, C leaves l1 and l2 = N/2
+    const bool skip_col = s != 0, skip_row = s == 2 && r == H;
+    cplx<T> x[H], o[H];
+    sfor<0, H>([&](auto K) {
+        const int c = 2 * int(K) + h;
+        const cplx<T> ec = ph[ca * N + c];
+        const cplx<T> v = erE * ec - ert * (c == H ? conj(ec) : ec); // 2i kap
+        T g = T(0.5) * (v.y + v.x);                                  // Re kap - Im kap
+        if (skip_row || (skip_col && c == H)) g = T(0);
+        const cplx<T> f = F[int(K) * 2 * N];
+        x[K] = mk(g * (f.x + f.y), g * (f.y - f.x));                 // (1 - i) g f
+    });
+    cplx<T>* P = L + s * N * PI;
+    pair_dft_dit<T, N, +1>(x, o, h);                                 // over the columns
+    sfor<0, H>([&](auto K) { P[r * PI + H * h + K] = o[K]; });
     __syncthreads();
-    lds_fft_row<T, N, +1>(P, c);          // over b for row c
-    __syncthreads();
-    lds_fft_col<T, N, +1>(P, c);          // over a for column c
-    __syncthreads();
-    // stores (coalesced): A[y][z] = P[y][z]; B[z][x] = P[x][z]; C[y][x] = P[x][y]
-    T* dst = nyq + ((((size_t(t) * NW + w) * Nrho + p) * M + q) * 6 + slot) * NN;
-    sfor<0, N>([&](auto K) {
-        constexpr int k = K;
-        dst[k * N + c] = (type == 0) ? P[k * (N + 1) + c].y : P[c * (N + 1) + k].y;
+    sfor<0, H>([&](auto K) { x[K] = P[(2 * int(K) + h) * PI + r]; });
+    pair_dft_dit<T, N, +1>(x, o, h);                                 // over the rows
+    T* dst = nyq + ((((size_t(t) * NW + w) * Nrho + p) * M + q) * 6 + 2 * s) * NN + r;
+    sfor<0, H>([&](auto K) {
+        dst[(H * h + int(K)) * N] = o[K].x;                          // beta
+        dst[NN + (H * h + int(K)) * N] = o[K].y;                     // delta
     });
 }
 
@@ -257,6 +267,54 @@ struct NyLayout {
     static constexpr int B = 2 * N * NS;          // [sgn][j][x]  (pitch BP)
     static constexpr int C = B + 2 * NS * BP;     // [sgn][y][x]  (pitch BP)
     static constexpr int SIZE = C + 2 * N * BP;
+};
+
+// Staging of a (task, p, q)'s Nyquist data for residue r by NT threads: item
+// i = A+- [y][j], B+- [j][x], C+- [y][x] of the NW functions in turn.  load()
+// issues all of a thread's loads, store() puts them into the LDS image, so
+// that one memory latency and not one per item is paid (and none where the
+// loads are issued a pass ahead).
+template <typename T, int N, int S, int NW, int NT>
+struct NyStage {
+    using NL = NyLayout<N, S>;
+    static constexpr int NS = N / S, NN = N * N, BP = NL::BP;
+    static constexpr int PER = 4 * N * NS + 2 * NN, ITEMS = NW * PER, K = (ITEMS + NT - 1) / NT;
+    T v[K];
+    // src: this (t, w = 0, p, q)'s planes; wstride: from one function's to the next
+    DGFS_DEV void load(const T* src, size_t wstride, int r) {
+        sfor<0, K>([&](auto Ki) {
+            const int i = int(threadIdx.x) + int(Ki) * NT;
+            if (i >= ITEMS) return;
+            const int w = NW == 1 ? 0 : i / PER, k = NW == 1 ? i : i - w * PER;
+            const T* s = src + w * wstride;
+            if (k < 2 * N * NS) {                        // A: e = y NS + j
+                const int sg = k / (N * NS), e = k - sg * N * NS;
+                v[Ki] = s[sg * NN + (e / NS) * N + S * (e % NS) + r];
+            } else if (k < 4 * N * NS) {                 // B: e = j N + x
+                const int k2 = k - 2 * N * NS, sg = k2 / (N * NS), e = k2 - sg * N * NS;
+                v[Ki] = s[(2 + sg) * NN + (S * (e / N) + r) * N + e % N];
+            } else {                                     // C: e = y N + x
+                v[Ki] = s[4 * NN + k - 4 * N * NS];
+            }
+        });
+    }
+    DGFS_DEV void store(T* Ny) const {
+        sfor<0, K>([&](auto Ki) {
+            const int i = int(threadIdx.x) + int(Ki) * NT;
+            if (i >= ITEMS) return;
+            const int w = NW == 1 ? 0 : i / PER, k = NW == 1 ? i : i - w * PER;
+            T* d = Ny + w * NL::SIZE;
+            if (k < 2 * N * NS) {
+                d[NL::A + k] = v[Ki];
+            } else if (k < 4 * N * NS) {
+                const int k2 = k - 2 * N * NS, sg = k2 / (N * NS), e = k2 - sg * N * NS;
+                d[NL::B + sg * NS * BP + (e / N) * BP + e % N] = v[Ki];
+            } else {
+                const int k2 = k - 4 * N * NS, sg = k2 / NN, e = k2 - sg * NN;
+                d[NL::C + sg * N * BP + (e / N) * BP + e % N] = v[Ki];
+            }
+        });
+    }
 };
 
 template <typename T, int N, int S>
@@ -386,34 +444,10 @@ k_gain(const cplx<T>* __restrict__ Fhat, const cplx<T>* __restrict__ phase,
                 [&] {
                     if constexpr (wv != 0) return;
                     // stage this q's Nyquist imaginary parts for residue r
-                    for (int i = threadIdx.x; i < NW * 6 * N * NS + NW * 2 * NN;
-                         i += E::NT) {
-                        if (i < NW * 6 * N * NS) {
-                            // A+- [y][j] and B+- [j][x] (both N*NS per sign)
-                            const int w = i / (6 * N * NS), k = i - w * 6 * N * NS;
-                            const int seg = k / (N * NS), e = k - seg * (N * NS);  // seg 0..5
-                            if (seg >= 4) continue;
-                            const T* src = nyq + ((((size_t(t) * NW + w) * Nrho + p) * M + q) * 6 +
-                                                  seg) * NN;
-                            T* dstw = Ny + w * NL::SIZE;
-                            if (seg < 2) {       // A: e = y*NS + j
-                                const int y = e / NS, j = e - y * NS;
-                                dstw[NL::A + seg * N * NS + e] = src[y * N + S * j + r];
-                            } else {             // B: e = j*N + x
-                                const int j = e / N, x = e - j * N;
-                                dstw[NL::B + (seg - 2) * NS * BP + j * BP + x] =
-                                    src[(S * j + r) * N + x];
-                            }
-                        } else {
-                            // C+- [y][x]
-                            const int k0 = i - NW * 6 * N * NS;
-                            const int w = k0 / (2 * NN), k = k0 - w * 2 * NN;
-                            const int sg = k / NN, e = k - sg * NN;
-                            const T* src = nyq + ((((size_t(t) * NW + w) * Nrho + p) * M + q) * 6 +
-                                                  4 + sg) * NN;
-                            Ny[w * NL::SIZE + NL::C + sg * N * BP + (e / N) * BP + e % N] = src[e];
-                        }
-                    }
+                    NyStage<T, N, S, NW, E::NT> st;
+                    st.load(nyq + ((size_t(t) * NW * Nrho + p) * M + q) * 6 * NN,
+                            size_t(Nrho) * M * 6 * NN, r);
+                    st.store(Ny);
                 },
                 map1,
                 [&](int i1, int i2, int i3) {
@@ -551,37 +585,22 @@ k_gain_pair(const cplx<T>* __restrict__ Fhat, const cplx<T>* __restrict__ phase,
     auto map1 = [](int pp, int& i1, int& i2) { i1 = pp / N; i2 = pp - (pp / N) * N; };  // (l1, l2)
     auto map3 = [](int Q, int& o2, int& j) { o2 = Q / NS; j = Q - (Q / NS) * NS; };      // (y, j)
 
+    // the next q's Nyquist data is loaded while this one's passes 2 and 3 run:
+    // one work-group fills a CU, so nothing else hides that latency (ahead of
+    // pass 1's loads it delayed them)
+    NyStage<T, N, S, 1, E::NT> stage;
+    const T* nyt = nyq + (size_t(t) * Nrho + p) * M * 6 * NN;
+    if (q0 < q1) stage.load(nyt + size_t(q0) * 6 * NN, 0, r);
     for (int q = q0; q < q1; ++q) {
         const cplx<T>* ph = phase + (size_t(p) * M + q) * 3 * N;   // [axis][l]
         const cplx<T>* pzq = phz + (size_t(p) * M + q) * N;          // [l3]
         // pass 1 reads F[l3][l1][l2] at the pencil's lane offset plus a
         // compile-time plane offset
         const auto Fb = buffer_view(Ff, unsigned(n * sizeof(cplx<T>)));
-        auto prologue = [&] {
-                // stage this q's Nyquist imaginary parts for residue r
-                for (int i = threadIdx.x; i < 6 * N * NS + 2 * NN; i += E::NT) {
-                    if (i < 6 * N * NS) {
-                        // A+- [y][j] and B+- [j][x] (both N*NS per sign)
-                        const int seg = i / (N * NS), e = i - seg * (N * NS);   // seg 0..5
-                        if (seg >= 4) continue;
-                        const T* src = nyq + (((size_t(t) * Nrho + p) * M + q) * 6 + seg) * NN;
-                        if (seg < 2) {       // A: e = y*NS + j
-                            const int y = e / NS, j = e - y * NS;
-                            Ny[NL::A + seg * N * NS + e] = src[y * N + S * j + r];
-                        } else {             // B: e = j*N + x
-                            const int j = e / N, x = e - j * N;
-                            Ny[NL::B + (seg - 2) * NS * BP + j * BP + x] =
-                                src[(S * j + r) * N + x];
-                        }
-                    } else {
-                        // C+- [y][x]
-                        const int k = i - 6 * N * NS;
-                        const int sg = k / NN, e = k - sg * NN;
-                        const T* src = nyq + (((size_t(t) * Nrho + p) * M + q) * 6 + 4 + sg) * NN;
-                        Ny[NL::C + sg * N * BP + (e / N) * BP + e % N] = src[e];
-                    }
-                }
-            };
+        auto prologue = [&] { stage.store(Ny); };
+        auto mid = [&] {
+            if (q + 1 < q1) stage.load(nyt + size_t(q + 1) * 6 * NN, 0, r);
+        };
         auto load = [&](int i1, int i2, int i3) {
                 // Re e + Im e of e = ph_x ph_y ph_z from the z factors' pair
                 const cplx<T> a = ph[i1] * ph[N + i2], z = pzq[i3];
@@ -651,7 +670,7 @@ k_gain_pair(const cplx<T>* __restrict__ Fhat, const cplx<T>* __restrict__ phase,
         // the residue r is uniform per work-group: one instantiation per r, so
         // that the engine's split twiddles are compile-time constants
         sfor<0, S>([&](auto Ri) {
-            if (r == int(Ri)) E::template run<int(Ri)>(V, prologue, map1, load, map3, epi);
+            if (r == int(Ri)) E::template run<int(Ri)>(V, prologue, map1, load, mid, map3, epi);
         });
     }
     if constexpr (MODE == kGainStore) return;
@@ -898,6 +917,7 @@ struct CollisionPlan {
     void* acc = nullptr;    // [ntask][Nrho][QG][n] cplx<T>
     void* Iw = nullptr;     // [ntask][2][n] cplx<T>  forward-transform intermediate
     void* H = nullptr;      // [ntask][2][n] cplx<T>  plane-inverted loss / gain
+    void* FN = nullptr;     // [ntask][2][3][N*N] cplx<T>  Nyquist planes of the last F^
     void* nyq = nullptr;    // [ntask][2][Nrho][M][6][N*N] T  Nyquist-plane imaginary parts
     // reference-state form: F0^ ([ntask][2][n] cplx<T>, slot 0 used) and
     // u+-_f0 ([ntask][Nrho][M][n] UPair<T>) of the reference state, valid for
@@ -960,7 +980,7 @@ struct Impl {
         if (int rc = forward(pl, u, ug, tv, ntask, nfg, dev, (cplx<T>*)pl->Fhat, st)) return rc;
         timing_mark(pl, 1, st);
         hipLaunchKernelGGL((k_nyq<T, N>), dim3(ntask * nfg * pl->Nrho * pl->M), dim3(6 * N), 0,
-                           st, (const cplx<T>*)pl->Fhat, (const cplx<T>*)pl->phase, pl->M,
+                           st, (const cplx<T>*)pl->FN, (const cplx<T>*)pl->phase, pl->M,
                            pl->Nrho, nfg, (T*)pl->nyq);
         DGFS_HIP_CHECK(hipGetLastError());
         timing_mark(pl, 2, st);
@@ -1054,7 +1074,7 @@ struct Impl {
         DGFS_HIP_CHECK(hipGetLastError());
         const long nli = long(ntask) * nfg * NN;
         hipLaunchKernelGGL((k_fwd_line<T, N>), dim3((nli + 255) / 256), dim3(256), 0, st, nli,
-                           nfg, (const cplx<T>*)pl->Iw, dst);
+                           nfg, (const cplx<T>*)pl->Iw, dst, (cplx<T>*)pl->FN);
         DGFS_HIP_CHECK(hipGetLastError());
         return 0;
     }
@@ -1065,7 +1085,7 @@ struct Impl {
                              hipStream_t st) {
         if (int rc = forward(pl, u0, u0, tv, ntask, 1, false, (cplx<T>*)pl->Fhat0, st)) return rc;
         hipLaunchKernelGGL((k_nyq<T, N>), dim3(ntask * pl->Nrho * pl->M), dim3(6 * N), 0, st,
-                           (const cplx<T>*)pl->Fhat0, (const cplx<T>*)pl->phase, pl->M, pl->Nrho,
+                           (const cplx<T>*)pl->FN, (const cplx<T>*)pl->phase, pl->M, pl->Nrho,
                            1, (T*)pl->nyq);
         DGFS_HIP_CHECK(hipGetLastError());
         const int nb = ntask * pl->Nrho * S1 * pl->QG;

@@ -388,13 +388,15 @@ struct Fft3Pair : Fft3Engine<T, N_, S_, 2 * N_ * (N_ / S_), DIR_, PAD> {
         pair_dft_dit<T, N, DIR>(x, o, h);
     }
 
-    template <int R, class Pro, class Map1, class Load, class Map3, class Epi>
-    static DGFS_DEV void run(cplx<T>* V, Pro&& prologue, Map1&& map1, Load&& load, Map3&& map3,
-                             Epi&& epi) {
+    // mid() runs by every thread between passes 1 and 2, behind pass 1's loads
+    template <int R, class Pro, class Map1, class Load, class Mid, class Map3, class Epi>
+    static DGFS_DEV void run(cplx<T>* V, Pro&& prologue, Map1&& map1, Load&& load, Mid&& mid,
+                             Map3&& map3, Epi&& epi) {
         __syncthreads();
         prologue();
         pass1<R>(V, map1, load);
         __syncthreads();
+        mid();
         pass2(V);
         __syncthreads();
         int o2, j;

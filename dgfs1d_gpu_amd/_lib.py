@@ -84,6 +84,7 @@ SIGNATURES = {
     'dgfs_collision_plan_query': (_i, [_vp, _ip, _ip, _ip, _szp]),
     'dgfs_collision_plan_set_qgroups': (_i, [_vp, _i]),
     'dgfs_collision_plan_set_schedule': (_i, [_vp, _i, _i]),
+    'dgfs_collide_pairs': (_i, [_vp, _vp, _vp, _i, _i, _i, _i, _vp, _vp, _vp, _i] + [_vp] * 9),
     'dgfs_collide': (_i, [_vp, _vp, _vp, _vp, _i, _i, _i, _vp, _vp, _vp, _i, _vp, _vp, _i,
                           _vp]),
     'dgfs_collision_reference_set': (_i, [_vp, _vp, _i, _i, _i, _vp, _vp, _vp, _vp]),

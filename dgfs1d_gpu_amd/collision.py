@@ -57,6 +57,66 @@ def task_table(K, Ne, tasks, tdtype, device):
         gslice=torch.tensor(np.array(gslice, np.int32), device=device))
 
 
+# tasks x points x directions x radii of a right-hand side from which the pair
+# form pays (its gain, plane and Nyquist stages are two launches each).  Tasks
+# against pairs in us, M = 12, N_rho = 8, modal bases: 18.4 M (N = 20, FP32, 24
+# tasks) 232/250; 18.1 M (N = 16, FP32, 46) 151/134; 31.5 M (N = 16, FP32, 80)
+# 197/149; 31.9 M (N = 24, FP32, 24) 452/383; 106 M (N = 24, FP32, 80) 1287/679;
+# 145 M (N = 32, FP64, 46) 11771/5324.
+PAIR_WORK = 20 << 20
+
+
+def pair_table(K, Ne, tasks, tdtype, device):
+    """Device tables of dgfs_collide_pairs for a list of tasks, or None where the
+    tasks themselves need no more transforms.  A task costs one transform per
+    direction when every task has f = g and two otherwise; a pair (b, b) one, a
+    pair (a, b) two."""
+    import torch
+    out = {}
+    for o, fterms, gterms in tasks:
+        T = out.setdefault(o, {})
+        for a, ca in fterms:
+            for b, cb in gterms:
+                T[a, b] = T.get((a, b), 0.0) + ca * cb
+    for T in out.values():                     # what is left of exact zeros
+        most = max((abs(v) for v in T.values()), default=0.0)
+        for ab in [ab for ab, v in T.items() if abs(v) <= 1e-15 * most]:
+            del T[ab]
+    diag = sorted({b for T in out.values() for _, b in T})
+    off = sorted({(min(ab), max(ab)) for T in out.values() for ab in T if ab[0] != ab[1]})
+    same = all(sorted(f) == sorted(g) for _, f, g in tasks)
+    if not diag or len(diag) + 2 * len(off) > 0.8 * len(tasks) * (1 if same else 2):
+        return None
+    pairs = [(b, b) for b in diag] + off
+    index = {ab: t for t, ab in enumerate(pairs)}
+    gs, gp, gc, ls, lp, lsl, lc = [0], [], [], [0], [], [], []
+    for o in sorted(out):
+        T = out[o]
+        sym = {}
+        for (a, b), v in T.items():
+            k = (min(a, b), max(a, b))
+            sym[k] = sym.get(k, 0.0) + v
+        for k in sorted(sym):
+            gp.append(index[k])
+            gc.append(sym[k])
+        gs.append(len(gp))
+        for a, b in sorted(T, key=lambda ab: (ab[1], ab[0])):
+            lp.append(index[b, b])
+            lsl.append(a)
+            lc.append(T[a, b])
+        ls.append(len(lp))
+    sl = np.zeros((len(pairs), 2, K), np.int32)
+    cf = np.zeros((len(pairs), 2, K), np.float64)
+    sl[:, 0, 0], sl[:, 1, 0] = np.array(pairs).T
+    cf[:, :, 0] = 1.0
+    ints = lambda x: torch.tensor(np.asarray(x, np.int32), device=device)
+    vals = lambda x: torch.tensor(np.asarray(x, np.float64), dtype=tdtype, device=device)
+    return dict(npair=len(pairs), ndiag=len(diag), nout=len(out),
+                nterm=ints(np.ones((len(pairs), 2))), slice=ints(sl), coef=vals(cf),
+                oslice=ints(sorted(out)), gstart=ints(gs), gpair=ints(gp), gcoef=vals(gc),
+                lstart=ints(ls), lpair=ints(lp), lslice=ints(lsl), lcoef=vals(lc))
+
+
 class CollisionPlan:
     def __init__(self, N, M, Nrho, L, qz, qw, sz, sw, gamma, prefac, dtype, variant,
                  ntask_max, device='cuda'):
@@ -82,6 +142,7 @@ class CollisionPlan:
         self._h = h
         self.ntask_max = int(ntask_max)
         self.tasks = None
+        self.pairs = None
 
     def query(self):
         s, qg, pg = _lib.C.c_int(), _lib.C.c_int(), _lib.C.c_int()
@@ -107,6 +168,11 @@ class CollisionPlan:
         if len(tasks) > self.ntask_max:
             raise ValueError('too many collision tasks (%d > %d)' % (len(tasks), self.ntask_max))
         self.tasks = task_table(K, Ne, tasks, self.tdtype, self.device)
+        self.pairs = None
+        if self.variant == _lib.VHS and len(tasks) * self.M * self.Nrho * self.n >= PAIR_WORK:
+            pairs = pair_table(K, Ne, tasks, self.tdtype, self.device)
+            if pairs is not None and pairs['npair'] <= self.ntask_max:
+                self.pairs = pairs
         return self.tasks
 
     def __call__(self, u, Q, stream=None, ug=None, tasks=None):
@@ -124,6 +190,15 @@ class CollisionPlan:
         n = t['K'] * t['Ne'] * self.n
         if u.numel() < n or Q.numel() < n or (ug is not None and ug.numel() < n):
             raise ValueError('collision operands smaller than K*Ne*Nv')
+        if tasks is None and ug is None and self.pairs is not None:
+            p = self.pairs
+            _lib.check(_lib.lib().dgfs_collide_pairs(
+                self._h, _lib.ptr(u), _lib.ptr(Q), t['K'], t['Ne'], p['npair'], p['ndiag'],
+                _lib.ptr(p['nterm']), _lib.ptr(p['slice']), _lib.ptr(p['coef']), p['nout'],
+                _lib.ptr(p['oslice']), _lib.ptr(p['gstart']), _lib.ptr(p['gpair']),
+                _lib.ptr(p['gcoef']), _lib.ptr(p['lstart']), _lib.ptr(p['lpair']),
+                _lib.ptr(p['lslice']), _lib.ptr(p['lcoef']), _lib.stream_ptr(stream)))
+            return
         fg_same = t['fg_same'] if ug is None else 0
         _lib.check(_lib.lib().dgfs_collide(
             self._h, _lib.ptr(u), _lib.ptr(ug), _lib.ptr(Q), t['K'], t['Ne'], t['ntask'],

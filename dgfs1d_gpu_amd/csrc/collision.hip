@@ -65,6 +65,26 @@ static int dispatch_reference_set(CollisionPlan* pl, const void* u0, TaskView tv
     return 2;
 }
 
+template <typename T>
+static int dispatch_pairs(CollisionPlan* pl, const void* u, void* Q, TaskView tv, int npair,
+                          int ndiag, PairOutput po, int nout, hipStream_t st) {
+#define DGFS_CASE(NN)                                                                     \
+    case NN:                                                                              \
+        return pairs_launch<T, NN>(pl, u, Q, tv, npair, ndiag, po, nout, st);
+    switch (pl->N) {
+        DGFS_CASE(4) DGFS_CASE(6) DGFS_CASE(8) DGFS_CASE(12) DGFS_CASE(16) DGFS_CASE(20)
+        DGFS_CASE(24) DGFS_CASE(32)
+        case 48:
+            if constexpr (std::is_same<T, float>::value)
+                return pairs_launch<T, 48>(pl, u, Q, tv, npair, ndiag, po, nout, st);
+            break;
+        default: break;
+    }
+#undef DGFS_CASE
+    set_error("collision: unsupported velocity grid N=%d", pl->N);
+    return 2;
+}
+
 static bool supported_N(int N) {
     return N == 4 || N == 6 || N == 8 || N == 12 || N == 16 || N == 20 || N == 24 || N == 32 ||
            N == 48;
@@ -310,6 +330,34 @@ extern "C" int dgfs_collide(dgfs_collision_plan_t plan, const void* u, const voi
                                       group_slice, fg_same, stream, nullptr);
     return dgfs::dispatch<float>(pl, u, ug, Q, tv, ntask, ngroup, group_start, group_slice,
                                  fg_same, stream, nullptr);
+}
+
+extern "C" int dgfs_collide_pairs(dgfs_collision_plan_t plan, const void* u, void* Q, int K, int Ne,
+                                  int npair, int ndiag, const int* pair_nterm,
+                                  const int* pair_slice, const void* pair_coef, int nout,
+                                  const int* out_slice, const int* gain_start,
+                                  const int* gain_pair, const void* gain_coef,
+                                  const int* loss_start, const int* loss_pair,
+                                  const int* loss_slice, const void* loss_coef,
+                                  hipStream_t stream) {
+    auto* pl = static_cast<CollisionPlan*>(plan);
+    DGFS_REQUIRE(pl, "collide_pairs: null plan");
+    DGFS_REQUIRE(npair >= 0 && npair <= pl->ntask_max, "collide_pairs: npair=%d exceeds plan max %d",
+                 npair, pl->ntask_max);
+    DGFS_REQUIRE(ndiag >= 0 && ndiag <= npair && (npair == 0 || ndiag > 0),
+                 "collide_pairs: bad ndiag=%d", ndiag);
+    DGFS_REQUIRE(K > 0 && Ne > 0 && nout >= 0, "collide_pairs: bad K/Ne/nout");
+    DGFS_REQUIRE(pl->variant == DGFS_VHS, "collide_pairs: vhs-gll evaluates Q(f, f) only");
+    if (npair == 0 || nout == 0) return 0;
+    DGFS_REQUIRE(u && Q && pair_nterm && pair_slice && pair_coef && out_slice && gain_start &&
+                     gain_pair && gain_coef && loss_start && loss_pair && loss_slice && loss_coef,
+                 "collide_pairs: null pointer argument");
+    dgfs::TaskView tv{K, Ne, int(pl->n), pair_nterm, pair_slice, pair_coef};
+    const dgfs::PairOutput po{gain_start, gain_pair, gain_coef, loss_start, loss_pair, loss_slice,
+                              loss_coef, out_slice};
+    if (pl->dtype == DGFS_F64)
+        return dgfs::dispatch_pairs<double>(pl, u, Q, tv, npair, ndiag, po, nout, stream);
+    return dgfs::dispatch_pairs<float>(pl, u, Q, tv, npair, ndiag, po, nout, stream);
 }
 
 extern "C" int dgfs_collision_reference_set(dgfs_collision_plan_t plan, const void* u0, int K,

@@ -898,6 +898,68 @@ k_line_output(const T* __restrict__ u, const T* __restrict__ u0, const double* _
     }
 }
 
+// ================================================== pair form of a right-hand side
+// Where the tasks couple modes (Q_m = sum_ab T_m,ab Q(u_a, u_b)), the gains of
+// the distinct unordered pairs {a, b} and the losses of the distinct b serve
+// every output slice: pair tasks t < ndiag are (b, b) (one transform per
+// direction; their loss is L[u_b]), the others (a, b), a != b (two).
+struct PairOutput {
+    const int* gstart;      // [nout + 1]  gain entries of an output
+    const int* gtask;       // pair task of an entry
+    const void* gcoef;      // its coefficient: T_ab + T_ba, or T_aa
+    const int* lstart;      // [nout + 1]  loss entries, those of one task together
+    const int* ltask;       // the (b, b) task
+    const int* lslice;      // a
+    const void* lcoef;      // T_ab
+    const int* oslice;      // [nout]  output slice
+};
+
+// Q[oslice[o]] += prefac (Re IFFT_k1 sum_j gcoef_j Hg[gtask_j]
+//                         - sum_j lcoef_j u[lslice_j] Re IFFT_k1 Hl[ltask_j])
+template <typename T, int N>
+__global__ void __launch_bounds__(kLineWG)
+k_line_pairs(const T* __restrict__ u, const cplx<T>* __restrict__ H, long nlines, PairOutput po,
+             T prefac, T* __restrict__ Q) {
+    constexpr int NN = N * N, n = N * NN, LN = line_lanes(N), PN = N / LN;
+    const long tid = long(blockIdx.x) * kLineWG + threadIdx.x;
+    const long gid = tid / LN;
+    const int h = LN == 2 ? int(tid & 1) : 0;
+    if (gid >= nlines) return;
+    const int g = int(gid / NN), yz = int(gid - long(g) * NN), x0 = PN * h;
+    auto kin = [&](int k) { return LN == 2 ? 2 * k + h : k; };
+    auto inverse = [&](const cplx<T>* a, cplx<T>* o) {
+        if constexpr (LN == 2)
+            pair_dft_dit<T, N, +1>(a, o, h);
+        else
+            RegDFT<T, N, +1>::template run<1, 0>(a, o);
+    };
+    cplx<T> a[PN], o[PN];
+    T loss[PN];
+    sfor<0, PN>([&](auto I) { loss[I] = T(0); });
+    int have = -1;
+    for (int j = po.lstart[g]; j < po.lstart[g + 1]; ++j) {
+        const int t = po.ltask[j];
+        if (t != have) {
+            const cplx<T>* hl = H + size_t(t) * 2 * n + yz;
+            sfor<0, PN>([&](auto K) { a[K] = hl[size_t(kin(K)) * NN]; });
+            inverse(a, o);
+            have = t;
+        }
+        const T c = static_cast<const T*>(po.lcoef)[j];
+        const T* p = u + size_t(po.lslice[j]) * n + size_t(x0) * NN + yz;
+        sfor<0, PN>([&](auto X) { loss[X] += c * p[size_t(X) * NN] * o[X].x; });
+    }
+    sfor<0, PN>([&](auto I) { a[I] = mk(T(0), T(0)); });
+    for (int j = po.gstart[g]; j < po.gstart[g + 1]; ++j) {
+        const T c = static_cast<const T*>(po.gcoef)[j];
+        const cplx<T>* hg = H + (size_t(po.gtask[j]) * 2 + 1) * n + yz;
+        sfor<0, PN>([&](auto K) { a[K] = a[K] + c * hg[size_t(kin(K)) * NN]; });
+    }
+    inverse(a, o);
+    T* dst = Q + size_t(po.oslice[g]) * n + size_t(x0) * NN + yz;
+    sfor<0, PN>([&](auto X) { dst[size_t(X) * NN] += prefac * (o[X].x - loss[X]); });
+}
+
 // ================================================================ the plan
 struct CollisionPlan {
     int N, M, Nrho, dtype, variant, ntask_max, ngroup_max;
@@ -979,53 +1041,27 @@ struct Impl {
         timing_mark(pl, 0, st);
         if (int rc = forward(pl, u, ug, tv, ntask, nfg, dev, (cplx<T>*)pl->Fhat, st)) return rc;
         timing_mark(pl, 1, st);
-        hipLaunchKernelGGL((k_nyq<T, N>), dim3(ntask * nfg * pl->Nrho * pl->M), dim3(6 * N), 0,
-                           st, (const cplx<T>*)pl->FN, (const cplx<T>*)pl->phase, pl->M,
-                           pl->Nrho, nfg, (T*)pl->nyq);
-        DGFS_HIP_CHECK(hipGetLastError());
+        if (int rc = nyquist(pl, 0, ntask, nfg, st)) return rc;
         timing_mark(pl, 2, st);
-        const bool alt = fg_same && !dev && pl->gain_smul == 2 && S1x != S1;
-        const bool pair = fg_same && !alt && (kPair || kPair64);
-        const int S = alt ? S1x : (pair && !dev ? SP : (fg_same ? S1 : S2));
-        const int nb = ntask * pl->Nrho * S * pl->QG;
-        const int rm = pl->gain_remap;
+        int S = S1;
         if (dev) {
+            const int nb = ntask * pl->Nrho * S1 * pl->QG;
             if constexpr (kPair)
                 hipLaunchKernelGGL((k_gain_pair<T, N, S1, kGainDelta>), dim3(nb),
                                    dim3(2 * N * (N / S1)), 0, st, (const cplx<T>*)pl->Fhat,
                                    (const cplx<T>*)pl->phase, (const cplx<T>*)pl->phz,
-                                   (const T*)pl->nyq, pl->M, pl->Nrho,
-                                   pl->QG, (cplx<T>*)pl->acc, (UPair<T>*)pl->ucache, rm);
+                                   (const T*)pl->nyq, pl->M, pl->Nrho, pl->QG, (cplx<T>*)pl->acc,
+                                   (UPair<T>*)pl->ucache, pl->gain_remap);
             else
                 hipLaunchKernelGGL((k_gain<T, N, S1, 1, kGainDelta>), dim3(nb),
                                    dim3(round64(N * (N / S1))), 0, st, (const cplx<T>*)pl->Fhat,
                                    (const cplx<T>*)pl->phase, (const T*)pl->nyq, pl->M, pl->Nrho,
-                                   pl->QG, (cplx<T>*)pl->acc, (UPair<T>*)pl->ucache, rm);
-        } else if (pair) {
-            if constexpr (kPair || kPair64)
-                hipLaunchKernelGGL((k_gain_pair<T, N, SP, kGainAccumulate, PADP>), dim3(nb),
-                                   dim3(2 * N * (N / SP)), 0, st, (const cplx<T>*)pl->Fhat,
-                                   (const cplx<T>*)pl->phase, (const cplx<T>*)pl->phz,
-                                   (const T*)pl->nyq, pl->M, pl->Nrho,
-                                   pl->QG, (cplx<T>*)pl->acc, (UPair<T>*)nullptr, rm);
+                                   pl->QG, (cplx<T>*)pl->acc, (UPair<T>*)pl->ucache,
+                                   pl->gain_remap);
+            DGFS_HIP_CHECK(hipGetLastError());
+        } else if (int rc = gain(pl, 0, ntask, fg_same, &S, st)) {
+            return rc;
         }
-        else if (alt)
-            hipLaunchKernelGGL((k_gain<T, N, S1x, 1, kGainAccumulate, 0>), dim3(nb),
-                               dim3(round64(N * (N / S1x))), 0,
-                               st, (const cplx<T>*)pl->Fhat, (const cplx<T>*)pl->phase,
-                               (const T*)pl->nyq, pl->M, pl->Nrho, pl->QG, (cplx<T>*)pl->acc,
-                               (UPair<T>*)nullptr, rm);
-        else if (fg_same)
-            hipLaunchKernelGGL((k_gain<T, N, S1, 1>), dim3(nb), dim3(round64(N * (N / S1))), 0,
-                               st, (const cplx<T>*)pl->Fhat, (const cplx<T>*)pl->phase,
-                               (const T*)pl->nyq, pl->M, pl->Nrho, pl->QG, (cplx<T>*)pl->acc,
-                               (UPair<T>*)nullptr, rm);
-        else
-            hipLaunchKernelGGL((k_gain<T, N, S2, 2>), dim3(nb), dim3(round64(N * (N / S2))), 0,
-                               st, (const cplx<T>*)pl->Fhat, (const cplx<T>*)pl->phase,
-                               (const T*)pl->nyq, pl->M, pl->Nrho, pl->QG, (cplx<T>*)pl->acc,
-                               (UPair<T>*)nullptr, rm);
-        DGFS_HIP_CHECK(hipGetLastError());
         timing_mark(pl, 3, st);
         if (dev)
             hipLaunchKernelGGL((k_plane_weight<T, N, true>), dim3(ntask * (N / 2 + 1)),
@@ -1033,12 +1069,8 @@ struct Impl {
                                (const cplx<T>*)pl->acc, (const T*)pl->wtab,
                                (const cplx<T>*)pl->Fhat, (const cplx<T>*)pl->Fhat0,
                                (const T*)pl->bb2, fg_same, pl->Nrho, pl->QG, S, (cplx<T>*)pl->H);
-        else
-            hipLaunchKernelGGL((k_plane_weight<T, N, false>), dim3(ntask * (N / 2 + 1)),
-                               dim3(PL * N), 0,
-                               st, (const cplx<T>*)pl->acc, (const T*)pl->wtab,
-                               (const cplx<T>*)pl->Fhat, (const cplx<T>*)nullptr,
-                               (const T*)pl->bb2, fg_same, pl->Nrho, pl->QG, S, (cplx<T>*)pl->H);
+        else if (int rc = plane(pl, 0, ntask, fg_same, S, st))
+            return rc;
         DGFS_HIP_CHECK(hipGetLastError());
         timing_mark(pl, 4, st);
         const long nlo = long(ngroup) * NN;
@@ -1051,6 +1083,88 @@ struct Impl {
             hipLaunchKernelGGL((k_line_output<T, N, false>), dim3(nlb), dim3(kLineWG), 0, st,
                                (const T*)u, (const T*)ug, Q0, tv, (const cplx<T>*)pl->H, nlo,
                                gstart, gslice, T(pl->prefac), (T*)Q);
+        DGFS_HIP_CHECK(hipGetLastError());
+        timing_mark(pl, 5, st);
+        if (pl->ev && pl->ev_used < pl->ev_max) ++pl->ev_used;
+        return 0;
+    }
+
+    // the direct gain of cnt tasks from task t0 on; *S: the residue split of acc
+    static int gain(CollisionPlan* pl, int t0, int cnt, int fg_same, int* S, hipStream_t st) {
+        const bool alt = fg_same && pl->gain_smul == 2 && S1x != S1;
+        const bool pair = fg_same && !alt && (kPair || kPair64);
+        *S = alt ? S1x : (pair ? SP : (fg_same ? S1 : S2));
+        const dim3 nb(cnt * pl->Nrho * *S * pl->QG);
+        const int rm = pl->gain_remap, M = pl->M, Nrho = pl->Nrho, QG = pl->QG;
+        const cplx<T>* F = (const cplx<T>*)pl->Fhat + size_t(t0) * 2 * pl->n;
+        const cplx<T>* ph = (const cplx<T>*)pl->phase;
+        const T* ny = (const T*)pl->nyq + size_t(t0) * 2 * Nrho * M * 6 * N * N;
+        cplx<T>* acc = (cplx<T>*)pl->acc + size_t(t0) * Nrho * QG * pl->n;
+        if (pair) {
+            if constexpr (kPair || kPair64)
+                hipLaunchKernelGGL((k_gain_pair<T, N, SP, kGainAccumulate, PADP>), nb,
+                                   dim3(2 * N * (N / SP)), 0, st, F, ph, (const cplx<T>*)pl->phz,
+                                   ny, M, Nrho, QG, acc, (UPair<T>*)nullptr, rm);
+        } else if (alt) {
+            hipLaunchKernelGGL((k_gain<T, N, S1x, 1, kGainAccumulate, 0>), nb,
+                               dim3(round64(N * (N / S1x))), 0, st, F, ph, ny, M, Nrho, QG, acc,
+                               (UPair<T>*)nullptr, rm);
+        } else if (fg_same) {
+            hipLaunchKernelGGL((k_gain<T, N, S1, 1>), nb, dim3(round64(N * (N / S1))), 0, st, F,
+                               ph, ny, M, Nrho, QG, acc, (UPair<T>*)nullptr, rm);
+        } else {
+            hipLaunchKernelGGL((k_gain<T, N, S2, 2>), nb, dim3(round64(N * (N / S2))), 0, st, F,
+                               ph, ny, M, Nrho, QG, acc, (UPair<T>*)nullptr, rm);
+        }
+        DGFS_HIP_CHECK(hipGetLastError());
+        return 0;
+    }
+
+    // the plane stage of those tasks
+    static int plane(CollisionPlan* pl, int t0, int cnt, int fg_same, int S, hipStream_t st) {
+        hipLaunchKernelGGL((k_plane_weight<T, N, false>), dim3(cnt * (N / 2 + 1)), dim3(PL * N), 0,
+                           st, (const cplx<T>*)pl->acc + size_t(t0) * pl->Nrho * pl->QG * pl->n,
+                           (const T*)pl->wtab, (const cplx<T>*)pl->Fhat + size_t(t0) * 2 * pl->n,
+                           (const cplx<T>*)nullptr, (const T*)pl->bb2, fg_same, pl->Nrho, pl->QG, S,
+                           (cplx<T>*)pl->H + size_t(t0) * 2 * pl->n);
+        DGFS_HIP_CHECK(hipGetLastError());
+        return 0;
+    }
+
+    // Nyquist planes of nw functions of those tasks
+    static int nyquist(CollisionPlan* pl, int t0, int cnt, int nw, hipStream_t st) {
+        hipLaunchKernelGGL((k_nyq<T, N>), dim3(cnt * nw * pl->Nrho * pl->M), dim3(6 * N), 0, st,
+                           (const cplx<T>*)pl->FN + size_t(t0) * 2 * 3 * N * N,
+                           (const cplx<T>*)pl->phase, pl->M, pl->Nrho, nw,
+                           (T*)pl->nyq + size_t(t0) * 2 * pl->Nrho * pl->M * 6 * N * N);
+        DGFS_HIP_CHECK(hipGetLastError());
+        return 0;
+    }
+
+    // the pair form: ndiag tasks (b, b), then npair - ndiag tasks (a, b)
+    static int launch_pairs(CollisionPlan* pl, const void* u, void* Q, TaskView tv, int npair,
+                            int ndiag, PairOutput po, int nout, hipStream_t st) {
+        const int noff = npair - ndiag;
+        timing_mark(pl, 0, st);
+        if (int rc = forward(pl, u, u, tv, npair, 2, false, (cplx<T>*)pl->Fhat, st)) return rc;
+        timing_mark(pl, 1, st);
+        if (int rc = nyquist(pl, 0, ndiag, 1, st)) return rc;
+        if (noff)
+            if (int rc = nyquist(pl, ndiag, noff, 2, st)) return rc;
+        timing_mark(pl, 2, st);
+        int Sd = 1, So = 1;
+        if (int rc = gain(pl, 0, ndiag, 1, &Sd, st)) return rc;
+        if (noff)
+            if (int rc = gain(pl, ndiag, noff, 0, &So, st)) return rc;
+        timing_mark(pl, 3, st);
+        if (int rc = plane(pl, 0, ndiag, 1, Sd, st)) return rc;
+        if (noff)
+            if (int rc = plane(pl, ndiag, noff, 0, So, st)) return rc;
+        timing_mark(pl, 4, st);
+        const long nlo = long(nout) * N * N;
+        hipLaunchKernelGGL((k_line_pairs<T, N>),
+                           dim3((nlo * line_lanes(N) + kLineWG - 1) / kLineWG), dim3(kLineWG), 0,
+                           st, (const T*)u, (const cplx<T>*)pl->H, nlo, po, T(pl->prefac), (T*)Q);
         DGFS_HIP_CHECK(hipGetLastError());
         timing_mark(pl, 5, st);
         if (pl->ev && pl->ev_used < pl->ev_max) ++pl->ev_used;
@@ -1084,10 +1198,7 @@ struct Impl {
     static int reference_set(CollisionPlan* pl, const void* u0, TaskView tv, int ntask,
                              hipStream_t st) {
         if (int rc = forward(pl, u0, u0, tv, ntask, 1, false, (cplx<T>*)pl->Fhat0, st)) return rc;
-        hipLaunchKernelGGL((k_nyq<T, N>), dim3(ntask * pl->Nrho * pl->M), dim3(6 * N), 0, st,
-                           (const cplx<T>*)pl->FN, (const cplx<T>*)pl->phase, pl->M, pl->Nrho,
-                           1, (T*)pl->nyq);
-        DGFS_HIP_CHECK(hipGetLastError());
+        if (int rc = nyquist(pl, 0, ntask, 1, st)) return rc;
         const int nb = ntask * pl->Nrho * S1 * pl->QG;
         // the store pass lays the pairs out for the delta kernel that reads them
         if constexpr (kPair)
@@ -1113,6 +1224,12 @@ int reference_set_launch(CollisionPlan* pl, const void* u0, TaskView tv, int nta
 }
 
 template <typename T, int N>
+int pairs_launch(CollisionPlan* pl, const void* u, void* Q, TaskView tv, int npair, int ndiag,
+                 PairOutput po, int nout, hipStream_t st) {
+    return Impl<T, N>::launch_pairs(pl, u, Q, tv, npair, ndiag, po, nout, st);
+}
+
+template <typename T, int N>
 int collide_launch(CollisionPlan* pl, const void* u, const void* ug, void* Q, TaskView tv,
                    int ntask, int ngroup, const int* gs, const int* gsl, int fgs, hipStream_t st,
                    const double* Q0) {
@@ -1123,12 +1240,16 @@ int collide_launch(CollisionPlan* pl, const void* u, const void* ug, void* Q, Ta
     extern template int collide_launch<T, N>(CollisionPlan*, const void*, const void*, void*, \
                                              TaskView, int, int, const int*, const int*, int, \
                                              hipStream_t, const double*);                     \
+    extern template int pairs_launch<T, N>(CollisionPlan*, const void*, void*, TaskView, int, int, \
+                                           PairOutput, int, hipStream_t);                    \
     extern template int reference_set_launch<T, N>(CollisionPlan*, const void*, TaskView, int, \
                                                    hipStream_t);
 #define DGFS_COLLIDE_INST(T, N)                                                          \
     template int collide_launch<T, N>(CollisionPlan*, const void*, const void*, void*,     \
                                       TaskView, int, int, const int*, const int*, int,     \
                                       hipStream_t, const double*);                         \
+    template int pairs_launch<T, N>(CollisionPlan*, const void*, void*, TaskView, int, int, \
+                                    PairOutput, int, hipStream_t);                         \
     template int reference_set_launch<T, N>(CollisionPlan*, const void*, TaskView, int,    \
                                             hipStream_t);
 #define DGFS_COLLIDE_SIZES(X, T) X(T, 4) X(T, 6) X(T, 8) X(T, 12) X(T, 16) X(T, 20) X(T, 24) X(T, 32)

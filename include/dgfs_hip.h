@@ -95,6 +95,26 @@ int dgfs_collide(dgfs_collision_plan_t plan, const void* u, const void* ug, void
                  int ngroup, const int* group_start, const int* group_slice, int fg_same,
                  hipStream_t stream);
 
+/* The same right-hand side by distinct pairs of slices, for task tables that
+ * couple modes: with T_o,ab = sum over the tasks of output o of
+ * coef_f[a] coef_g[b],
+ *     Q[out_slice[o]] += prefac (sum_{a <= b} S_o,ab Gain(u_a, u_b)
+ *                                - sum_ab T_o,ab u_a Loss(u_b)),
+ * S_o,ab = T_o,ab + T_o,ba (a < b) or T_o,aa: the gain is a symmetric bilinear
+ * form, so the gains of the distinct pairs and the losses of the distinct
+ * slices serve every output.  Pair task t has the terms of dgfs_collide's
+ * tasks with one term each: t < ndiag are (b, b), the others (a, b), a != b.
+ * gain_start [nout+1], gain_pair, gain_coef: the pairs of an output and S;
+ * loss_start [nout+1], loss_pair (a (b, b) task; those of one task
+ * consecutive), loss_slice (a), loss_coef (T).  DGFS_VHS plans; distinct
+ * outputs have distinct slices.  Device arrays; coefficients in the dtype. */
+int dgfs_collide_pairs(dgfs_collision_plan_t plan, const void* u, void* Q, int K, int Ne,
+                       int npair, int ndiag, const int* pair_nterm, const int* pair_slice,
+                       const void* pair_coef, int nout, const int* out_slice,
+                       const int* gain_start, const int* gain_pair, const void* gain_coef,
+                       const int* loss_start, const int* loss_pair, const int* loss_slice,
+                       const void* loss_coef, hipStream_t stream);
+
 /* Reference-state form of the same collision (no counterpart in the
  * reference, whose fs() is FP64 end to end; it replaces dgfs_collide for
  * f = g tasks when the plan computes in FP32).  With f_t the task's f

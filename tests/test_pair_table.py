@@ -1,0 +1,85 @@
+"""The pair form of mode-coupling task tables (collision.pair_table) on the
+host: the gain and loss coefficients add up to the tasks' bilinear form over
+every accepted table, and tables that gain nothing keep their tasks."""
+import numpy as np
+import pytest
+
+from dgfs1d_gpu_amd.collision import pair_table
+
+
+def _forms(p, nsl):
+    """(symmetric gain form, loss form) per output from the tables."""
+    import torch
+    v = {k: (x.numpy() if isinstance(x, torch.Tensor) else x) for k, x in p.items()}
+    first = v['slice'][:, 0, 0], v['slice'][:, 1, 0]
+    assert (v['nterm'] == 1).all() and (v['coef'][:, :, 0] == 1.0).all()
+    assert (first[0][:v['ndiag']] == first[1][:v['ndiag']]).all()
+    assert (first[0][v['ndiag']:] != first[1][v['ndiag']:]).all()
+    out = {}
+    for o in range(v['nout']):
+        G, L = np.zeros((nsl, nsl)), np.zeros((nsl, nsl))
+        for j in range(v['gstart'][o], v['gstart'][o + 1]):
+            a, b = first[0][v['gpair'][j]], first[1][v['gpair'][j]]
+            G[a, b] += v['gcoef'][j] / 2
+            G[b, a] += v['gcoef'][j] / 2
+        last = []
+        for j in range(v['lstart'][o], v['lstart'][o + 1]):
+            t = v['lpair'][j]
+            assert t < v['ndiag']
+            if not last or last[-1] != t:
+                assert t not in last           # one task's entries are consecutive
+                last.append(t)
+            L[v['lslice'][j], first[1][t]] += v['lcoef'][j]
+        out[int(v['oslice'][o])] = G, L
+    return out
+
+
+def _check(K, Ne, tasks):
+    import torch
+    p = pair_table(K, Ne, tasks, torch.float64, 'cpu')
+    assert p is not None
+    nsl = K * Ne
+    ref = {}
+    for o, f, g in tasks:
+        T = ref.setdefault(o, np.zeros((nsl, nsl)))
+        for a, ca in f:
+            for b, cb in g:
+                T[a, b] += ca * cb
+    got = _forms(p, nsl)
+    assert set(got) == set(ref)
+    for o, T in ref.items():
+        tol = 1e-14 * np.abs(T).max()
+        assert np.abs(got[o][1] - T).max() <= tol
+        assert np.abs(got[o][0] - (T + T.T) / 2).max() <= tol
+    return p
+
+
+@pytest.mark.parametrize('K', [2, 3, 4, 5, 7])
+@pytest.mark.parametrize('kind', ['modal-orthonormal-legendre', 'modal-modified-karniadakis'])
+def test_modal_bases(K, kind):
+    from dgfs1d_gpu_amd.basis import Basis
+    from dgfs1d_gpu_amd.dictionary import Dictionary
+    from dgfs1d_gpu_amd.nputil import subclass_where
+    cfg = Dictionary('[basis]\nkind = %s\nK = %d\nNqr = 4\n' % (kind, K))
+    tasks = subclass_where(Basis, basis_kind=kind)(cfg).collision_tasks(3)
+    p = _check(K, 3, tasks)
+    assert p['ndiag'] == 3 * K and p['npair'] <= len(tasks)
+
+
+def test_unsymmetric_and_repeated_terms():
+    """f and g of different slices, repeated slices in a task, outputs that
+    share pairs, an output whose terms cancel."""
+    tasks = [(0, [(0, 1.0), (1, -2.0)], [(1, 0.5), (0, 1.5)]), (0, [(1, 1.0)], [(0, 3.0)]),
+             (2, [(0, 1.0), (0, 1.0)], [(1, 1.0)]), (2, [(1, 0.25)], [(0, 1.0)]),
+             (1, [(0, 1.0)], [(0, 1.0)]), (3, [(1, 1.0)], [(1, 1.0)]),
+             (3, [(1, -1.0)], [(1, 1.0)])]
+    _check(2, 2, tasks)
+
+
+def test_tables_without_gain_keep_their_tasks():
+    import torch
+    nodal = [(s, [(s, 1.0)], [(s, 1.0)]) for s in range(6)]
+    assert pair_table(3, 2, nodal, torch.float64, 'cpu') is None
+    cross = [(0, [(0, 1.0)], [(1, 1.0)]), (1, [(2, 1.0)], [(3, 1.0)])]
+    assert pair_table(2, 2, cross, torch.float64, 'cpu') is None
+    assert pair_table(2, 2, [], torch.float64, 'cpu') is None

@@ -12,13 +12,35 @@ import numpy as np
 from . import _lib
 
 
+def _bilinear_forms(tasks):
+    """{output slice: {(a, b): sum over its tasks of coef_f[a] coef_g[b]}}."""
+    out = {}
+    for o, fterms, gterms in tasks:
+        T = out.setdefault(o, {})
+        for a, ca in fterms:
+            for b, cb in gterms:
+                T[a, b] = T.get((a, b), 0.0) + ca * cb
+    return out
+
+
+def _symmetric(tasks):
+    """Whether the tasks of every output slice add up to a form symmetric in f
+    and g, to FP64 rounding."""
+    for T in _bilinear_forms(tasks).values():
+        most = max((abs(v) for v in T.values()), default=0.0)
+        if any(not abs(v - T.get((b, a), 0.0)) <= 1e-14 * most for (a, b), v in T.items()):
+            return False
+    return True
+
+
 def task_table(K, Ne, tasks, tdtype, device):
     """Device task table shared by the collision and relaxation entry points.
 
     tasks: (out_slice, f_terms, g_terms) with terms [(slice, coef), ...]; the
     table is sorted by output slice and grouped (one group per distinct output
     slice): nterm [T][2], slice [T][2][K], coef [T][2][K] (tdtype), group_start
-    [G+1], group_slice [G], and fg_same = every task has identical f and g terms."""
+    [G+1], group_slice [G], fg_same = every task has identical f and g terms, and
+    symmetric = the tasks of each output slice add up to a symmetric form."""
     import torch
     tasks = sorted(tasks, key=lambda t: t[0])
     T = len(tasks)
@@ -50,6 +72,7 @@ def task_table(K, Ne, tasks, tdtype, device):
         gslice.append(tasks[-1][0])
     return dict(
         K=int(K), Ne=int(Ne), ntask=T, ngroup=len(gslice), fg_same=int(fg_same),
+        symmetric=fg_same or _symmetric(tasks),
         nterm=torch.tensor(nterm, dtype=torch.int32, device=device),
         slice=torch.tensor(sl, dtype=torch.int32, device=device),
         coef=torch.tensor(cf, dtype=tdtype, device=device),
@@ -72,12 +95,7 @@ def pair_table(K, Ne, tasks, tdtype, device):
     direction when every task has f = g and two otherwise; a pair (b, b) one, a
     pair (a, b) two."""
     import torch
-    out = {}
-    for o, fterms, gterms in tasks:
-        T = out.setdefault(o, {})
-        for a, ca in fterms:
-            for b, cb in gterms:
-                T[a, b] = T.get((a, b), 0.0) + ca * cb
+    out = _bilinear_forms(tasks)
     for T in out.values():                     # what is left of exact zeros
         most = max((abs(v) for v in T.values()), default=0.0)
         for ab in [ab for ab, v in T.items() if abs(v) <= 1e-15 * most]:
@@ -332,8 +350,8 @@ class BiCollisionPlan:
         n = t['K'] * t['Ne'] * self.n
         if min(up.numel(), uq.numel(), Q.numel()) < n:
             raise ValueError('collision operands smaller than K*Ne*Nv')
-        if t['fg_same'] and up.data_ptr() == uq.data_ptr():
-            # a species with itself, f = g in every task
+        if t['symmetric'] and up.data_ptr() == uq.data_ptr():
+            # a species with itself
             _lib.check(_lib.lib().dgfs_bi_collide_like(
                 self._h, _lib.ptr(up), _lib.ptr(Q), t['K'], t['Ne'], t['ntask'],
                 _lib.ptr(t['nterm']), _lib.ptr(t['slice']), _lib.ptr(t['coef']), t['ngroup'],

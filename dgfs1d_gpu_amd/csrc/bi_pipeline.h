@@ -28,9 +28,10 @@
 //   k2 = N/2 and k3 = N/2 of every x-plane travel as extra pencils, and
 //   k1 = N/2 is the plane transform of sum_x (-1)^x Im P.
 // * For an antipodally symmetric direction rule (and pre-rule)
-//   W_-s = conj W_s, so an opposite pair shares one weight; and when f = g
-//   with equal masses u1 and u2 swap under s -> -s, so the pair shares its
-//   product: one product per pair with the weight 2 Re W.
+//   W_-s = conj W_s, so an opposite pair shares one weight; and with equal
+//   masses P_-s(f, g) = P_s(g, f), so where an output's tasks add up to a form
+//   symmetric in f and g (a species with itself) the pair shares its product:
+//   one product per pair with the weight 2 Re W.
 //
 // Layouts: pencil p(l2, l3) = (l3 / 2) 2N + 2 l2 + (l3 & 1), the order in
 // which k_bi_plane's lanes hold a plane; F[which][l1][p]; Y[d][x][p];

@@ -270,7 +270,7 @@ int bi_stream_chunk(BiPlan* pl, int nt, bool like, cplx<T>* Z, hipStream_t st) {
     return 0;
 }
 
-// like: up = uq and every task's f and g terms are the same
+// like: up = uq and each output's tasks add up to a form symmetric in f and g
 template <typename T, int N>
 int bi_launch(BiPlan* pl, const void* up, const void* uq, void* Q, TaskView tv, int ntask,
               int ngroup, const int* gstart, const int* gslice, bool like, hipStream_t st) {

@@ -192,10 +192,12 @@ int dgfs_bi_collide(dgfs_bi_collision_plan_t plan, const void* up, const void* u
                     int K, int Ne, int ntask, const int* task_nterm, const int* task_slice,
                     const void* task_coef, int ngroup, const int* group_start,
                     const int* group_slice, hipStream_t stream);
-/* dgfs_bi_collide(plan, u, u, Q, ...) for task tables whose f and g terms are
- * the same in every task (a species with itself on a nodal basis).  With
- * equal masses and antipodally symmetric rules opposite directions share one
- * product, which halves the work; otherwise the same as dgfs_bi_collide. */
+/* dgfs_bi_collide(plan, u, u, Q, ...), a species with itself, for task tables
+ * whose tasks add up to a form symmetric in f and g for each output slice
+ * (equal terms, or all singular triplets of a symmetric coupling matrix).  With
+ * equal masses and antipodally symmetric rules the product of direction -s is
+ * that of s with f and g exchanged, so opposite directions share one product:
+ * half the work; otherwise the same as dgfs_bi_collide. */
 int dgfs_bi_collide_like(dgfs_bi_collision_plan_t plan, const void* u, void* Q, int K, int Ne,
                          int ntask, const int* task_nterm, const int* task_slice,
                          const void* task_coef, int ngroup, const int* group_start,

@@ -67,23 +67,38 @@ def test_rules(cuda, N, dtype, M, antipodal):
     assert err < (1e-11 if dtype == 'F64' else 3e-5)
 
 
+# singular triplets of symmetric 2 x 2 couplings (degenerate and not), and a
+# single-slice task with unequal coefficients
+TRIPLETS = [(0, [(0, 1.0)], [(1, 0.7)]), (0, [(1, 1.0)], [(0, 0.7)]),
+            (1, [(0, 0.8), (1, 0.6)], [(0, 0.8), (1, 0.6)]),
+            (1, [(0, -0.6), (1, 0.8)], [(0, 0.3), (1, -0.4)]), (3, [(2, 0.5)], [(2, 3.0)])]
 SAME = [(0, [(0, 1.0)], [(0, 1.0)]), (1, [(1, 0.5), (3, 0.25)], [(1, 0.5), (3, 0.25)]),
         (1, [(2, -1.0)], [(2, -1.0)])]
 
 
 @pytest.mark.parametrize('N,dtype', [(20, 'F64'), (24, 'F32'), (32, 'F64')])
 @pytest.mark.parametrize('M,antipodal', [(6, True), (5, False)])
-def test_like_species(cuda, N, dtype, M, antipodal):
-    """up is uq with equal f and g terms: one product per opposite pair; the
-    same task table with another array takes the general form."""
+@pytest.mark.parametrize('tasks', ['same', 'triplets'])
+def test_like_species(cuda, N, dtype, M, antipodal, tasks):
+    """up is uq and the tasks of each output symmetric in f and g: one product
+    per opposite pair; the same table with another array takes the general
+    form."""
     from dgfs1d_gpu_amd import _lib
     d = getattr(_lib, dtype)
-    a, err, _ = _call(cuda, N, M, antipodal, d, 1, 1, 400 // M, SAME, like=True)
-    b, _, _ = _call(cuda, N, M, antipodal, d, 1, 1, 400 // M, SAME, oracle=False)
+    todo = SAME if tasks == 'same' else TRIPLETS
+    a, err, _ = _call(cuda, N, M, antipodal, d, 1, 1, 400 // M, todo, like=True)
+    b, _, _ = _call(cuda, N, M, antipodal, d, 1, 1, 400 // M, todo, oracle=False)
     diff = np.abs(a - b).max() / np.abs(b).max()
     print(N, dtype, M, err, diff, flush=True)
     assert err < (1e-11 if dtype == 'F64' else 3e-5)
     assert diff < (1e-13 if dtype == 'F64' else 3e-5)
+
+
+def test_one_species_with_unsymmetric_tasks(cuda):
+    """up is uq, but f and g do not exchange: the general form."""
+    from dgfs1d_gpu_amd import _lib
+    a, err, _ = _call(cuda, 20, 6, True, _lib.F64, 0, 0, 70, TASKS, like=True)
+    assert err < 1e-11
 
 
 def test_like_call_of_unequal_masses(cuda):

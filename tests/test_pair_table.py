@@ -83,3 +83,23 @@ def test_tables_without_gain_keep_their_tasks():
     cross = [(0, [(0, 1.0)], [(1, 1.0)]), (1, [(2, 1.0)], [(3, 1.0)])]
     assert pair_table(2, 2, cross, torch.float64, 'cpu') is None
     assert pair_table(2, 2, [], torch.float64, 'cpu') is None
+
+
+def test_symmetric_flag():
+    """task_table marks exactly the tables whose outputs are symmetric in f and g."""
+    import torch
+    from dgfs1d_gpu_amd.basis import Basis
+    from dgfs1d_gpu_amd.collision import task_table
+    from dgfs1d_gpu_amd.dictionary import Dictionary
+    from dgfs1d_gpu_amd.nputil import subclass_where
+    flag = lambda K, Ne, t: task_table(K, Ne, t, torch.float64, 'cpu')['symmetric']
+    kind = 'modal-orthonormal-legendre'
+    for K in (2, 3, 5):
+        cfg = Dictionary('[basis]\nkind = %s\nK = %d\nNqr = 4\n' % (kind, K))
+        assert flag(K, 2, subclass_where(Basis, basis_kind=kind)(cfg).collision_tasks(2))
+    assert flag(2, 1, [(0, [(1, 0.5)], [(1, 2.0)])])
+    assert not flag(2, 1, [(0, [(0, 1.0)], [(1, 1.0)])])
+    both = [(0, [(0, 1.0)], [(1, 1.0)]), (0, [(1, 1.0)], [(0, 1.0)])]
+    assert flag(2, 1, both)
+    assert not flag(2, 1, [both[0], (1,) + both[1][1:]])
+    assert not flag(2, 1, [(0, [(0, float('nan'))], [(1, 1.0)])])

@@ -34,10 +34,12 @@
 //   one product per pair with the weight 2 Re W.
 //
 // Layouts: pencil p(l2, l3) = (l3 / 2) 2N + 2 l2 + (l3 & 1), the order in
-// which k_bi_plane's lanes hold a plane; F[which][l1][p]; Y[d][x][p];
-// acc[d][x][q] with q the regular pencils k3 <= N/2 (same formula), then the
-// lines (k2 = N/2, k3 = 0..N/2) and (k2, k3 = N/2); x = N .. N + XS - 1 are
-// the k1 = N/2 planes of the XS x-ranges.  Every length-N transform is shared
+// which k_bi_plane's lanes hold a plane; F[which][l1][p]; Y[d][x][p], whose
+// planes k_bi_plane overwrites with its results: Y[d][x][q], q < NPT <= N^2,
+// with q the regular pencils k3 <= N/2 (same formula), then the lines
+// (k2 = N/2, k3 = 0..N/2) and (k2, k3 = N/2).  In place a product takes 0.57
+// instead of 0.9 MB (FP64 N = 32), so a chunk of the scratch budget holds 1.6
+// times the tasks.  spec[d][s][q]: the k1 = N/2 plane of x-range s.  Every length-N transform is shared
 // by a lane pair (pair_dft_*): half the registers per lane.
 #pragma once
 #include "collision_kernels.h"
@@ -52,6 +54,7 @@ struct BiGeo {
     static constexpr int NE = H + 1 + N;            // line pencils
     static constexpr int NPT = NPH + NE;
     static_assert(N % 2 == 0 && N >= 4, "even grids");
+    static_assert(N < 20 || NPT <= NN, "a plane's results fit its place in Y");
     static DGFS_HD int pen(int l2, int l3) { return (l3 / 2) * 2 * N + 2 * l2 + (l3 & 1); }
 };
 constexpr int kBiXSMax = 12;                        // most x-ranges of a product
@@ -275,14 +278,15 @@ struct BiPlane {
 
 // Slot (t, d, s) takes x-range s of product d: per plane the inverses along
 // l3 and l2, the product, the forward transforms along y and z and the split
-// into R and the Nyquist lines of J.
+// into R and the Nyquist lines of J, over the plane it read: no other live slot
+// reads that plane, and the slot's lanes have theirs before the first barrier.
 template <typename T, int N>
 __global__ void __launch_bounds__((BiPlane<T, N>::WG), 2)
-k_bi_plane(const cplx<T>* __restrict__ Y, const cplx<T>* __restrict__ nyq, long nslot, int XS,
-           cplx<T>* __restrict__ acc) {
+k_bi_plane(cplx<T>* Y, const cplx<T>* __restrict__ nyq, long nslot, int XS,
+           cplx<T>* __restrict__ spec) {
     using Gm = BiGeo<N>;
     using Pl = BiPlane<T, N>;
-    constexpr int H = Gm::H, NN = Gm::NN, NPT = Gm::NPT, NPH = Gm::NPH;
+    constexpr int H = Gm::H, NN = Gm::NN, NPH = Gm::NPH;
     constexpr int PI = Pl::PI, PN = Pl::PN, PW = Pl::PW, MH = Pl::MH;
     __shared__ cplx<T> L[PW * Pl::ELEMS];
     __shared__ cplx<T> Cs[PW * N];                    // row x of C
@@ -296,11 +300,10 @@ k_bi_plane(const cplx<T>* __restrict__ Y, const cplx<T>* __restrict__ nyq, long 
     const int s = int(slot - td * XS);
     cplx<T>* P = L + sl * Pl::ELEMS;
     cplx<T>* Cr = Cs + sl * N;
-    const cplx<T>* Yp = Y + td * size_t(N) * NN;
+    cplx<T>* Yp = Y + td * size_t(N) * NN;
     const cplx<T>* A = nyq + td * size_t(3) * NN;
     const cplx<T>* B = A + NN;
     const cplx<T>* C = B + NN;
-    cplx<T>* out = acc + td * size_t(N + XS) * NPT;
     const int nx = N / XS, x0 = s * nx;
     const int rm = r ? N - r : 0;                     // row of -k2
     const T sz = (r & 1) ? T(-1) : T(1);              // (-1)^z of this column
@@ -340,7 +343,7 @@ k_bi_plane(const cplx<T>* __restrict__ Y, const cplx<T>* __restrict__ nyq, long 
         Pl::forward(a, o, h);                         // row k2 = r -> k3
         Pl::template exchange<PN, MH>(P, o, a, row_in, row_mirror);
         if (live) {
-            cplx<T>* dst = out + size_t(x) * NPT;
+            cplx<T>* dst = Yp + size_t(x) * NN;
             sfor<0, MH>([&](auto M) {
                 const int k3 = Pl::in(M, h);
                 const cplx<T> c = conj(a[M]);
@@ -359,7 +362,7 @@ k_bi_plane(const cplx<T>* __restrict__ Y, const cplx<T>* __restrict__ nyq, long 
     Pl::template exchange<PN, PN>(P, o, a, col_in, row_out);
     Pl::forward(a, o, h);
     if (live) {
-        cplx<T>* dst = out + size_t(N + s) * NPT;
+        cplx<T>* dst = spec + size_t(slot) * NPH;
         sfor<0, MH>([&](auto M) { dst[Gm::pen(r, Pl::in(M, h))] = mul_i<1>(o[M]); });
     }
 }
@@ -373,11 +376,11 @@ enum BiWeight { kBiComplex = 0, kBiPair = 1, kBiReal = 2 };
 constexpr int kBiSumWG = 64;
 template <typename T, int N, int MODE>
 __global__ void __launch_bounds__(kBiSumWG, 2)
-k_bi_sum(const cplx<T>* __restrict__ acc, const cplx<T>* __restrict__ wtab,
-         const cplx<T>* __restrict__ wspec, int nt, int ND, int XS, int NU, int XG, int QB,
+k_bi_sum(const cplx<T>* __restrict__ Y, const cplx<T>* __restrict__ spec,
+         const cplx<T>* __restrict__ wtab, const cplx<T>* __restrict__ wspec, int nt, int ND, int XS, int NU, int XG, int QB,
          cplx<T>* __restrict__ Gp) {
     using Gm = BiGeo<N>;
-    constexpr int H = Gm::H, NPT = Gm::NPT, NPH = Gm::NPH;
+    constexpr int H = Gm::H, NN = Gm::NN, NPT = Gm::NPT, NPH = Gm::NPH;
     constexpr int NP = MODE == kBiPair ? 2 : 1;
     // consecutive work-groups (one XCD) take the tasks of one weight block
     const int lb = xcd_remap(blockIdx.x, gridDim.x);
@@ -395,9 +398,10 @@ k_bi_sum(const cplx<T>* __restrict__ acc, const cplx<T>* __restrict__ wtab,
 #pragma unroll 1
         for (int sgn = 0; sgn < NP; ++sgn) {              // one product's pencil at a time
             const T cj = sgn ? T(-1) : T(1);              // the second one's weight is conj(W_u)
-            const cplx<T>* src = acc + (size_t(t) * ND + NP * u + sgn) * size_t(N + XS) * NPT + q;
+            const size_t td = size_t(t) * ND + NP * u + sgn;
+            const cplx<T>* src = Y + td * N * NN + q;
             cplx<T> a[H], o[H];
-            sfor<0, H>([&](auto K) { a[K] = src[size_t(H * h + int(K)) * NPT]; });
+            sfor<0, H>([&](auto K) { a[K] = src[size_t(H * h + int(K)) * NN]; });
             pair_dft_dif<T, N, -1>(a, o, h);
             sfor<0, H>([&](auto M) {
                 const cplx<T> v = w[size_t(int(M)) * NPT * 2];
@@ -408,7 +412,7 @@ k_bi_sum(const cplx<T>* __restrict__ acc, const cplx<T>* __restrict__ wtab,
             });
             if (q < NPH && h == (H & 1)) {
                 cplx<T> sp = mk(T(0), T(0));
-                for (int s = 0; s < XS; ++s) sp = sp + src[size_t(N + s) * NPT];
+                for (int s = 0; s < XS; ++s) sp = sp + spec[(td * XS + s) * NPH + q];
                 cplx<T> v = wspec[size_t(u) * NPH + q];
                 if constexpr (MODE == kBiReal) v = mk(v.x + v.x, T(0));
                 G[H / 2] = G[H / 2] + mk(v.x, cj * v.y) * sp;     // k1 = N/2

@@ -90,7 +90,7 @@ static int bi_for_grid(int N, Fn&& f) {
 
 static void bi_free(BiPlan* pl) {
     for (void* p : {pl->phase, pl->wtab, pl->wspec, pl->ctab, pl->Fhat, pl->Iw, pl->Y, pl->nyq,
-                    pl->acc, pl->H, pl->norm, pl->Gp})
+                    pl->spec, pl->acc, pl->H, pl->norm, pl->Gp})
         if (p) (void)hipFree(p);
     delete pl;
 }
@@ -100,8 +100,9 @@ struct BiSizes {
     size_t wtab = 0, wspec = 0;             // weight tables
     size_t Y = 0, nyq = 0, acc = 0;         // per task
     size_t group = 0;                       // one group's partial G^ of a task
-    int groups = 1;                         // groups that Gp holds
+    int groups = 1;                         // groups per task (streaming: BiPlan::ngrp in all)
     size_t ctab = 0;                        // c_pq
+    size_t spec = 0;                        // a plane of spec
 };
 template <int N>
 static BiSizes bi_sizes(bool stream, int NXY, int NU) {
@@ -112,9 +113,8 @@ static BiSizes bi_sizes(bool stream, int NXY, int NU) {
         z.wspec = size_t(NU) * Gm::NPH;
         z.Y = size_t(NXY) * Gm::n;
         z.nyq = size_t(NXY) * 3 * Gm::NN;
-        z.acc = size_t(NXY) * size_t(N + kBiXSMax) * Gm::NPT;
         z.group = size_t(N) * Gm::NPT;
-        z.groups = NU < 64 ? NU : 64;
+        z.spec = Gm::NPH;
         z.ctab = size_t(N) * Gm::NPH;
     } else {
         z.wtab = z.acc = size_t(NXY) * Gm::n;
@@ -149,7 +149,7 @@ static std::vector<int> opposite(const double* p, int n) {
 
 // scratch budget of the gain products: tasks are processed in chunks whose
 // [chunk][Nrho*M][n] complex products fit in it
-constexpr size_t kBiAccBudget = size_t(8) << 30;
+constexpr size_t kBiAccBudget = size_t(2) << 30;
 
 }  // namespace dgfs
 
@@ -236,8 +236,7 @@ extern "C" int dgfs_bi_collision_plan_create(int N, int M, int Nrho, double L, c
     pl->stream = stream;
     pl->antipodal = antipodal;
     const dgfs::BiSizes sizes = dgfs::bi_sizes_of(pl);
-    pl->xg_max = sizes.groups;
-    const size_t per_task = (sizes.Y + sizes.nyq + sizes.acc) * cs;
+    const size_t per_task = (sizes.Y + sizes.nyq + sizes.acc + size_t(NXY) * sizes.spec) * cs;
     size_t budget = dgfs::kBiAccBudget;
     if (const char* mb = std::getenv("DGFS_BI_SCRATCH_MB")) {
         const long v = std::atol(mb);
@@ -247,6 +246,22 @@ extern "C" int dgfs_bi_collision_plan_create(int N, int M, int Nrho, double L, c
     if (chunk < 1) chunk = 1;
     if (chunk > size_t(ntask_max)) chunk = size_t(ntask_max);
     pl->chunk = int(chunk);
+    // a call that shares products takes half of them per task
+    const size_t lchunk = stream && antipodal && mp == mq
+                              ? std::min(2 * chunk, size_t(ntask_max)) : chunk;
+    pl->like_chunk = int(lchunk);
+
+    pl->ngrp = chunk * size_t(sizes.groups);
+    if (stream) {
+        auto more = [&](auto zero) {
+            using T = decltype(zero);
+            return dgfs::bi_for_grid<T>(N, [&](auto g) {
+                if constexpr (dgfs::bi_streams(int(g))) dgfs::bi_stream_sizes<T, int(g)>(pl);
+                return 0;
+            });
+        };
+        (void)(dtype == DGFS_F64 ? more(0.0) : more(0.0f));
+    }
 
     void *d_fac = nullptr, *d_wx = nullptr, *d_wc = nullptr, *d_sp = nullptr, *d_B = nullptr,
          *d_Bs = nullptr, *d_yl = nullptr;
@@ -275,12 +290,13 @@ extern "C" int dgfs_bi_collision_plan_create(int N, int M, int Nrho, double L, c
         (sizes.Y && hipMalloc(&pl->Y, chunk * sizes.Y * cs) != hipSuccess) ||
         (sizes.nyq && hipMalloc(&pl->nyq, chunk * sizes.nyq * cs) != hipSuccess) ||
         hipMalloc(&pl->ctab, sizes.ctab * cs) != hipSuccess ||
-        hipMalloc(&pl->Fhat, chunk * 2 * n * cs) != hipSuccess ||
-        hipMalloc(&pl->Iw, chunk * 2 * n * cs) != hipSuccess ||
-        hipMalloc(&pl->norm, chunk * 2 * dgfs::bi_norm_blocks(N) * sizeof(double)) != hipSuccess ||
-        hipMalloc(&pl->acc, chunk * sizes.acc * cs) != hipSuccess ||
+        hipMalloc(&pl->Fhat, lchunk * 2 * n * cs) != hipSuccess ||
+        hipMalloc(&pl->Iw, lchunk * 2 * n * cs) != hipSuccess ||
+        hipMalloc(&pl->norm, lchunk * 2 * dgfs::bi_norm_blocks(N) * sizeof(double)) != hipSuccess ||
+        (sizes.acc && hipMalloc(&pl->acc, chunk * sizes.acc * cs) != hipSuccess) ||
+        (pl->nspec && hipMalloc(&pl->spec, pl->nspec * sizes.spec * cs) != hipSuccess) ||
         hipMalloc(&pl->H, size_t(ntask_max) * 2 * n * cs) != hipSuccess ||
-        hipMalloc(&pl->Gp, chunk * size_t(sizes.groups) * sizes.group * cs) != hipSuccess) {
+        hipMalloc(&pl->Gp, pl->ngrp * sizes.group * cs) != hipSuccess) {
         dgfs::set_error("bi_collision_plan_create: allocation failed");
         return fail(1);
     }
@@ -337,8 +353,9 @@ extern "C" int dgfs_bi_collision_plan_query(dgfs_bi_collision_plan_t plan, int* 
     if (chunk) *chunk = pl->chunk;
     if (scratch_bytes) {
         const dgfs::BiSizes z = dgfs::bi_sizes_of(pl);
-        *scratch_bytes = (size_t(pl->chunk) * (4 * pl->n + z.Y + z.nyq + z.acc +
-                                               size_t(z.groups) * z.group) +
+        *scratch_bytes = (size_t(pl->chunk) * (z.Y + z.nyq + z.acc) +
+                          size_t(pl->like_chunk) * 4 * pl->n +
+                          pl->nspec * z.spec + pl->ngrp * z.group +
                           size_t(pl->ntask_max) * 2 * pl->n) * cs;
     }
     return 0;

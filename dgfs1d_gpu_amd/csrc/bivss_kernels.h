@@ -195,31 +195,86 @@ constexpr int bi_xgroups_max(int NXY) { return (NXY + planes_per_wg(N) - 1) / pl
 
 // ================================================================ the plan
 struct BiPlan {
-    int N, M, Nrho, Mpre, dtype, ntask_max, chunk;
+    int N, M, Nrho, Mpre, dtype, ntask_max;
+    int chunk;              // tasks whose products the scratch holds
+    int like_chunk;         // the same for calls that share products (bi_launch)
     double prefac, mp, mq;
     size_t n;
     bool stream = false;    // the streaming kernels (bi_pipeline.h)
     bool antipodal = false; // the streaming form's products come in opposite pairs (2u, 2u + 1)
-    int xg_max = 1;         // groups of k_bi_sum that Gp holds
+    size_t nspec = 0;       // planes of spec
+    size_t ngrp = 0;        // partial G^ that Gp holds
     void* phase = nullptr;  // [Nrho*M][2][3][N] cplx<T>, in product order
     void* wtab = nullptr;   // [Nrho*M][k1][k2][k3] cplx<T>  qw sw / n * b_pq; streaming: k_bi_wtab
     void* wspec = nullptr;  // streaming: the weights at k1 = N/2 (k_bi_wtab)
     void* ctab = nullptr;   // [l1][l2][l3] cplx<T>  c_pq; streaming: k_bi_chtab
-    void* Fhat = nullptr;   // [chunk][2][n] cplx<T>
-    void* Iw = nullptr;     // [chunk][2][n] cplx<T>
-    void* Y = nullptr;      // streaming: [chunk][Nrho*M][n] cplx<T>
+    void* Fhat = nullptr;   // [like_chunk][2][n] cplx<T>
+    void* Iw = nullptr;     // [like_chunk][2][n] cplx<T>
+    void* Y = nullptr;      // streaming: [chunk][Nrho*M][n] cplx<T>, before and after k_bi_plane
     void* nyq = nullptr;    // streaming: [chunk][Nrho*M][3][N*N] cplx<T>
-    void* acc = nullptr;    // [chunk][Nrho*M][n] cplx<T>; streaming: [chunk][Nrho*M][N + XS][NPT]
+    void* spec = nullptr;   // streaming: [chunk][Nrho*M][XS][NPH] cplx<T>
+    void* acc = nullptr;    // [chunk][Nrho*M][n] cplx<T>
     void* H = nullptr;      // [ntask_max][2][n] cplx<T>: loss, gain
-    void* norm = nullptr;   // streaming: [chunk][2][bi_norm_blocks] FP64
-    void* Gp = nullptr;     // [chunk][groups][n] cplx<T>  partial G^; streaming: [..][H][NPT][2]
+    void* norm = nullptr;   // streaming: [like_chunk][2][bi_norm_blocks] FP64
+    void* Gp = nullptr;     // [chunk][groups][n] cplx<T>  partial G^; streaming: [ngrp][H][NPT][2]
 };
 
+// x-ranges of k_bi_plane and weight groups of k_bi_sum for nt tasks of ND
+// products, NU weights: the split with the shortest longest CU.  A CU's share
+// is its ceil(blocks / 256) work-groups, but no less than the eight waves that
+// it needs to be busy, times the length of one; finer splits even the shares
+// out and pay per piece (a range its k1 = N/2 plane, about half a plane's
+// transforms; a group the write and the read of its partial sums, about two
+// weights).  Against the first split of at least 2048 waves, same chunks: N = 20
+// FP64 8.11 -> 7.83 ms, N = 48 FP32 41.9 -> 38.0, N = 32 FP64 29.7 both, the
+// 6-task N = 24 set 536/538 us (at 4096 waves it took 591).
+constexpr int kBiCU = 256;
+inline double bi_share(long blocks, int wg, double length) {
+    const long per = (blocks + kBiCU - 1) / kBiCU;
+    return std::max(double(per), 512.0 / wg) * length;
+}
+template <typename T, int N>
+inline int bi_xranges(int nt, int ND) {
+    using Pl = BiPlane<T, N>;
+    int XS = 1;
+    double least = 0.0;
+    for (int d = 1; d <= kBiXSMax; ++d) {
+        if (N % d) continue;
+        const double c = bi_share((long(nt) * ND * d + Pl::PW - 1) / Pl::PW, Pl::WG, N / d + 0.5);
+        if (d == 1 || c < least) XS = d, least = c;
+    }
+    return XS;
+}
+template <int N>
+inline int bi_sum_groups(int nt, int NU) {
+    constexpr int QB = (BiGeo<N>::NPT + kBiSumWG / 2 - 1) / (kBiSumWG / 2);
+    int XG = 1;
+    double least = 0.0;
+    for (int per = NU; per >= 1; --per) {
+        const int g = (NU + per - 1) / per;
+        if (g > 64) break;
+        const double c = bi_share(long(nt) * QB * g, kBiSumWG, per + 2.0);
+        if (per == NU || c < least) XG = g, least = c;
+    }
+    return XG;
+}
+// the most planes of spec and partial sums of Gp that a chunk takes, with or
+// without the shared products of `like`
+template <typename T, int N>
+inline void bi_stream_sizes(BiPlan* pl) {
+    const int NXY = pl->Nrho * pl->M, us = pl->antipodal ? 2 : 1;
+    auto take = [&](int chunk, int ND) {
+        for (int nt = 1; nt <= chunk; ++nt) {
+            pl->nspec = std::max(pl->nspec, size_t(nt) * ND * bi_xranges<T, N>(nt, ND));
+            pl->ngrp = std::max(pl->ngrp, size_t(nt) * bi_sum_groups<N>(nt, NXY / us));
+        }
+    };
+    take(pl->chunk, NXY);
+    take(pl->like_chunk, NXY / us);
+}
+
 // The streaming form for nt tasks: forward plane transforms of f, g in Iw ->
-// the x-planes of loss and gain in Z.  The groups and ranges spread a small task set over the chip:
-// each kernel gets at least the 2048 waves that are resident at two per SIMD
-// where the task set allows it (finer groups reload F and G, more ranges add
-// their k1 = N/2 planes: twice the waves made the 6-task N = 24 set 8 % slower).
+// the x-planes of loss and gain in Z.
 template <typename T, int N>
 int bi_stream_chunk(BiPlan* pl, int nt, bool like, cplx<T>* Z, hipStream_t st) {
     using Gm = BiGeo<N>;
@@ -233,35 +288,29 @@ int bi_stream_chunk(BiPlan* pl, int nt, bool like, cplx<T>* Z, hipStream_t st) {
     hipLaunchKernelGGL((k_bi_fwd_line<T, N>), dim3(nt * 2 * bi_norm_blocks(N)), dim3(256), 0, st,
                        (const cplx<T>*)pl->Iw, (cplx<T>*)pl->Fhat, norm);
     DGFS_HIP_CHECK(hipGetLastError());
-    auto groups = [](long want, long have, int most) {
-        const long g = (want + have - 1) / have;
-        return int(g < 1 ? 1 : (g > most ? most : g));
-    };
     const int PB = (Gm::NN + kBiXWG / 2 - 1) / (kBiXWG / 2);
-    const int XGX = groups(2048, long(nt) * PB * (kBiXWG / 64), (ND + 1) / 2);
+    // 8192 waves (at 2048: N = 20 8.30, N = 32 30.4, N = 48 43.8 against 8.11, 29.7,
+    // 41.9 ms); a group reloads F and G, so it has two products or more
+    const long xb = long(nt) * PB * (kBiXWG / 64);
+    const int XGX = int(std::max(1L, std::min((8192 + xb - 1) / xb, long(ND + 1) / 2)));
     const int nxb = nt * PB * XGX;
     const long nny = long(nt) * ND * 3;
     constexpr int NPW = BiNyq<T, N>::PW;
     hipLaunchKernelGGL((k_bi_x<T, N>), dim3(nxb + (nny + NPW - 1) / NPW), dim3(kBiXWG), 0, st, F, ph,
                        norm, ND, dstride, PB, XGX, nxb, (cplx<T>*)pl->Y, nny, (cplx<T>*)pl->nyq);
     DGFS_HIP_CHECK(hipGetLastError());
-    int XS = 1;
-    for (int d = 2; d <= kBiXSMax; ++d)
-        if (N % d == 0 && long(nt) * ND * XS * Pl::PT / 64 < 2048) XS = d;
+    const int XS = bi_xranges<T, N>(nt, ND);
     const long ns = long(nt) * ND * XS;
     hipLaunchKernelGGL((k_bi_plane<T, N>), dim3((ns + Pl::PW - 1) / Pl::PW), dim3(Pl::WG), 0, st,
-                       (const cplx<T>*)pl->Y, (const cplx<T>*)pl->nyq, ns, XS, (cplx<T>*)pl->acc);
+                       (cplx<T>*)pl->Y, (const cplx<T>*)pl->nyq, ns, XS, (cplx<T>*)pl->spec);
     DGFS_HIP_CHECK(hipGetLastError());
     const int QB = (Gm::NPT + kBiSumWG / 2 - 1) / (kBiSumWG / 2);
-    // whole units per group; Gp holds chunk * xg_max groups
-    int XG = groups(2048, long(nt) * QB * (kBiSumWG / 64), NU);
-    XG = int(std::min<long>(XG, long(pl->xg_max) * pl->chunk / nt));
-    XG = (NU + (NU + XG - 1) / XG - 1) / ((NU + XG - 1) / XG);
+    const int XG = bi_sum_groups<N>(nt, NU);
     auto* sum = like ? k_bi_sum<T, N, kBiReal>
                      : (pl->antipodal ? k_bi_sum<T, N, kBiPair> : k_bi_sum<T, N, kBiComplex>);
-    hipLaunchKernelGGL(sum, dim3(nt * QB * XG), dim3(kBiSumWG), 0, st, (const cplx<T>*)pl->acc,
-                       (const cplx<T>*)pl->wtab, (const cplx<T>*)pl->wspec, nt, ND, XS, NU, XG, QB,
-                       (cplx<T>*)pl->Gp);
+    hipLaunchKernelGGL(sum, dim3(nt * QB * XG), dim3(kBiSumWG), 0, st, (const cplx<T>*)pl->Y,
+                       (const cplx<T>*)pl->spec, (const cplx<T>*)pl->wtab,
+                       (const cplx<T>*)pl->wspec, nt, ND, XS, NU, XG, QB, (cplx<T>*)pl->Gp);
     DGFS_HIP_CHECK(hipGetLastError());
     const int QF = (Gm::NPH + 31) / 32;
     hipLaunchKernelGGL((k_bi_pen<T, N>), dim3(nt * QF), dim3(kBiPenWG), 0, st, (const cplx<T>*)pl->Gp,
@@ -278,8 +327,12 @@ int bi_launch(BiPlan* pl, const void* up, const void* uq, void* Q, TaskView tv, 
     const int NXY = pl->Nrho * pl->M;
     const size_t n = pl->n;
     like = like && pl->antipodal && pl->mp == pl->mq;
-    for (int c0 = 0; c0 < ntask; c0 += pl->chunk) {
-        const int nt = ntask - c0 < pl->chunk ? ntask - c0 : pl->chunk;
+    // even chunks: a short last one would leave the chip idle at each kernel's end
+    const int most = like ? pl->like_chunk : pl->chunk;
+    const int nchunk = (ntask + most - 1) / most;
+    const int per = nchunk ? (ntask + nchunk - 1) / nchunk : 0;
+    for (int c0 = 0; c0 < ntask; c0 += per) {
+        const int nt = ntask - c0 < per ? ntask - c0 : per;
         TaskView tc = tv;
         tc.nterm = tv.nterm + 2 * size_t(c0);
         tc.slice = tv.slice + size_t(c0) * 2 * tv.K;

@@ -147,15 +147,22 @@ def test_trace_species(cuda, ratio):
     assert err < 3e-5
 
 
-def test_chunks(cuda, monkeypatch):
-    """One and two tasks per chunk (other group and x-range splits) change
-    nothing but the order of sums."""
+@pytest.mark.parametrize('like', [False, True])
+def test_chunks(cuda, monkeypatch, like):
+    """One and two tasks per chunk (twice that where a call shares products;
+    other group and x-range splits) change nothing but the order of sums."""
     from dgfs1d_gpu_amd import _lib
-    ref, _, info = _call(cuda, 32, 6, True, _lib.F64, 0, 1, len(TASKS), oracle=False)
+    todo = SAME * 2 if like else TASKS                # 10.5 MB of scratch per task
+    q = 0 if like else 1
+
+    def call(oracle):
+        return _call(cuda, 32, 6, True, _lib.F64, 0, q, len(todo), todo, like=like, oracle=oracle)
+    ref, err, info = call(True)
+    assert err < 1e-11
     seen = {info['chunk']}
-    for mb in ('1', '44'):
+    for mb in ('1', '22'):
         monkeypatch.setenv('DGFS_BI_SCRATCH_MB', mb)
-        got, _, info = _call(cuda, 32, 6, True, _lib.F64, 0, 1, len(TASKS), oracle=False)
+        got, _, info = call(False)
         seen.add(info['chunk'])
         assert np.abs(got - ref).max() < 1e-13 * np.abs(ref).max()
-    assert len(seen) == 3, seen
+    assert seen == {1, 2, len(todo)}, seen

@@ -281,38 +281,42 @@ struct NyStage {
     static constexpr int PER = 4 * N * NS + 2 * NN, ITEMS = NW * PER, K = (ITEMS + NT - 1) / NT;
     T v[K];
     // src: this (t, w = 0, p, q)'s planes; wstride: from one function's to the next
+    static DGFS_DEV T get(int i, const T* src, size_t wstride, int r) {
+        const int w = NW == 1 ? 0 : i / PER, k = NW == 1 ? i : i - w * PER;
+        const T* s = src + w * wstride;
+        if (k < 2 * N * NS) {                            // A: e = y NS + j
+            const int sg = k / (N * NS), e = k - sg * N * NS;
+            return s[sg * NN + (e / NS) * N + S * (e % NS) + r];
+        }
+        if (k < 4 * N * NS) {                            // B: e = j N + x
+            const int k2 = k - 2 * N * NS, sg = k2 / (N * NS), e = k2 - sg * N * NS;
+            return s[(2 + sg) * NN + (S * (e / N) + r) * N + e % N];
+        }
+        return s[4 * NN + k - 4 * N * NS];               // C: e = y N + x
+    }
+    static DGFS_DEV void put(int i, T x, T* Ny) {
+        const int w = NW == 1 ? 0 : i / PER, k = NW == 1 ? i : i - w * PER;
+        T* d = Ny + w * NL::SIZE;
+        if (k < 2 * N * NS) {
+            d[NL::A + k] = x;
+        } else if (k < 4 * N * NS) {
+            const int k2 = k - 2 * N * NS, sg = k2 / (N * NS), e = k2 - sg * N * NS;
+            d[NL::B + sg * NS * BP + (e / N) * BP + e % N] = x;
+        } else {
+            const int k2 = k - 4 * N * NS, sg = k2 / NN, e = k2 - sg * NN;
+            d[NL::C + sg * N * BP + (e / N) * BP + e % N] = x;
+        }
+    }
     DGFS_DEV void load(const T* src, size_t wstride, int r) {
         sfor<0, K>([&](auto Ki) {
             const int i = int(threadIdx.x) + int(Ki) * NT;
-            if (i >= ITEMS) return;
-            const int w = NW == 1 ? 0 : i / PER, k = NW == 1 ? i : i - w * PER;
-            const T* s = src + w * wstride;
-            if (k < 2 * N * NS) {                        // A: e = y NS + j
-                const int sg = k / (N * NS), e = k - sg * N * NS;
-                v[Ki] = s[sg * NN + (e / NS) * N + S * (e % NS) + r];
-            } else if (k < 4 * N * NS) {                 // B: e = j N + x
-                const int k2 = k - 2 * N * NS, sg = k2 / (N * NS), e = k2 - sg * N * NS;
-                v[Ki] = s[(2 + sg) * NN + (S * (e / N) + r) * N + e % N];
-            } else {                                     // C: e = y N + x
-                v[Ki] = s[4 * NN + k - 4 * N * NS];
-            }
+            if (i < ITEMS) v[Ki] = get(i, src, wstride, r);
         });
     }
     DGFS_DEV void store(T* Ny) const {
         sfor<0, K>([&](auto Ki) {
             const int i = int(threadIdx.x) + int(Ki) * NT;
-            if (i >= ITEMS) return;
-            const int w = NW == 1 ? 0 : i / PER, k = NW == 1 ? i : i - w * PER;
-            T* d = Ny + w * NL::SIZE;
-            if (k < 2 * N * NS) {
-                d[NL::A + k] = v[Ki];
-            } else if (k < 4 * N * NS) {
-                const int k2 = k - 2 * N * NS, sg = k2 / (N * NS), e = k2 - sg * N * NS;
-                d[NL::B + sg * NS * BP + (e / N) * BP + e % N] = v[Ki];
-            } else {
-                const int k2 = k - 4 * N * NS, sg = k2 / NN, e = k2 - sg * NN;
-                d[NL::C + sg * N * BP + (e / N) * BP + e % N] = v[Ki];
-            }
+            if (i < ITEMS) put(i, v[Ki], Ny);
         });
     }
 };
@@ -444,10 +448,21 @@ k_gain(const cplx<T>* __restrict__ Fhat, const cplx<T>* __restrict__ phase,
                 [&] {
                     if constexpr (wv != 0) return;
                     // stage this q's Nyquist imaginary parts for residue r
-                    NyStage<T, N, S, NW, E::NT> st;
-                    st.load(nyq + ((size_t(t) * NW * Nrho + p) * M + q) * 6 * NN,
-                            size_t(Nrho) * M * 6 * NN, r);
-                    st.store(Ny);
+                    // FP64 grids whose N^2 lanes do not fill their waves: item by
+                    // item (all of a thread's items in flight 81 against 76 us at
+                    // N = 12, 241 against 239 at N = 20; elsewhere they win: FP64
+                    // N = 16 88/95, N = 24 337/352, FP32 N = 20 147/157 us)
+                    using St = NyStage<T, N, S, NW, E::NT>;
+                    const T* src = nyq + ((size_t(t) * NW * Nrho + p) * M + q) * 6 * NN;
+                    const size_t ws = size_t(Nrho) * M * 6 * NN;
+                    if constexpr (sizeof(T) == 8 && N % 8 != 0) {
+                        for (int i = threadIdx.x; i < St::ITEMS; i += E::NT)
+                            St::put(i, St::get(i, src, ws, r), Ny);
+                    } else {
+                        St st;
+                        st.load(src, ws, r);
+                        st.store(Ny);
+                    }
                 },
                 map1,
                 [&](int i1, int i2, int i3) {

@@ -147,8 +147,9 @@ static std::vector<int> opposite(const double* p, int n) {
     return o;
 }
 
-// scratch budget of the gain products: tasks are processed in chunks whose
-// [chunk][Nrho*M][n] complex products fit in it
+// scratch budget of the gain products (streaming: with their Nyquist planes):
+// tasks are processed in chunks whose products fit in it.  Larger ones
+// (3 GiB and more) take up to seconds to allocate.
 constexpr size_t kBiAccBudget = size_t(2) << 30;
 
 }  // namespace dgfs

@@ -67,7 +67,10 @@ struct BiGeo {
 constexpr int kBiXSMax = 12;                        // most x-ranges of a product
 
 // F[t][which][k1][p] = FFT_x(Iw)/n, one thread per (t, which, p), and
-// norm[t][which][blk] = the work-group's sum of |F|^2.
+// norm[t][which][0][blk] = the work-group's sum of |F|^2, 0 only where F is zero.
+// FP64 sums whose squares could leave the range (FP32's fit an FP64 sum) are
+// taken again, scaled by the largest component: -s there and e in
+// norm[t][which][1][blk] stand for s 4^e.
 constexpr int bi_norm_blocks(int N) { return (N * N + 255) / 256; }
 template <typename T, int N>
 __global__ void __launch_bounds__(256)
@@ -76,45 +79,103 @@ k_bi_fwd_line(const cplx<T>* __restrict__ Iw, cplx<T>* __restrict__ F, double* _
     __shared__ double sh[4];
     const int blk = blockIdx.x % NB, tw = blockIdx.x / NB;
     const int p = blk * 256 + int(threadIdx.x);
+    const bool live = p < NN;
+    cplx<T>* dst = F + tw * size_t(N) * NN + p;
     double s = 0.0;
-    if (p < NN) {
+    if (live) {
         const int l3 = 2 * (p / (2 * N)) + (p & 1), l2 = (p % (2 * N)) >> 1;
         const cplx<T>* src = Iw + tw * size_t(N) * NN + l3 * N + l2;
         cplx<T> a[N], o[N];
         sfor<0, N>([&](auto X) { a[X] = src[size_t(X) * NN]; });
         RegDFT<T, N, -1>::template run<1, 0>(a, o);
         const T inv_n = T(1) / T(N * NN);
-        cplx<T>* dst = F + tw * size_t(N) * NN + p;
         sfor<0, N>([&](auto K1) {
             const cplx<T> v = inv_n * o[K1];
             dst[size_t(K1) * NN] = v;
             s += double(v.x) * double(v.x) + double(v.y) * double(v.y);
         });
     }
-    for (int o = 32; o; o >>= 1) s += __shfl_down(s, o);
-    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
-    __syncthreads();
-    if (threadIdx.x == 0) norm[blockIdx.x] = (sh[0] + sh[1]) + (sh[2] + sh[3]);
+    auto total = [&](double v) {
+        for (int o = 32; o; o >>= 1) v += __shfl_down(v, o);
+        if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
+        __syncthreads();
+        return (sh[0] + sh[1]) + (sh[2] + sh[3]);
+    };
+    s = total(s);
+    double* out = norm + size_t(tw) * 2 * NB + blk;
+    if constexpr (sizeof(T) == 8) if (!(s > 1e-200 && s < 1e200)) {
+        double m = 0.0;
+        if (live)
+            for (int k = 0; k < N; ++k) {
+                const cplx<T> v = dst[size_t(k) * NN];
+                m = fmax(m, fmax(fabs(v.x), fabs(v.y)));
+            }
+        for (int o = 32; o; o >>= 1) m = fmax(m, __shfl_xor(m, o));
+        __syncthreads();
+        if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = m;
+        __syncthreads();
+        m = fmax(fmax(sh[0], sh[1]), fmax(sh[2], sh[3]));
+        const int e = m > 0.0 && !isinf(m) ? max(ilogb(m), -1000) : 0;   // 2^-e is finite
+        const double r = ldexp(1.0, -e);
+        s = 0.0;
+        if (live)
+            for (int k = 0; k < N; ++k) {
+                const cplx<T> v = r * dst[size_t(k) * NN];
+                s += v.x * v.x + v.y * v.y;
+            }
+        __syncthreads();
+        s = -total(s);
+        if (threadIdx.x == 0) out[NB] = double(e);
+    }
+    if (threadIdx.x == 0) *out = s;
 }
 
-// The power of two nearest |f| / |g| of task t: the two sides share one complex
-// transform, whose rounding is relative to the larger of them, so G enters
-// scaled to F's size and the gain is scaled back (both exactly).  1 where
-// either side is zero or not finite.
+// The two sides of task t share one complex transform, whose rounding is
+// relative to the larger of them: F enters as 2^f F and G as 2^g G (the factors
+// go with the phases), of sizes near 1 and at most a factor of 2 apart, and the
+// gain is multiplied by 2^-(f + g).  All three are exact, so each side keeps the
+// range and the relative precision of a transform of its own.  zero: a side is
+// exactly zero (and the other finite), and so is the gain, which the shared
+// transform would leave at the other side's rounding (eps |g|^2).  Sides that
+// are not finite enter as they are.
+struct BiScale {
+    int f, g;
+    bool zero;
+};
 template <typename T, int N>
-DGFS_DEV T bi_scale(const double* norm, int t) {
+DGFS_DEV BiScale bi_scale(const double* norm, int t) {
     constexpr int NB = bi_norm_blocks(N);
-    const double* p = norm + size_t(t) * 2 * NB;
-    double f = 0.0, g = 0.0;
-    for (int i = 0; i < NB; ++i) {
-        f += p[i];
-        g += p[NB + i];
+    const double* p = norm + size_t(t) * 4 * NB;
+    double s[2];
+    int e[2];
+    for (int w = 0; w < 2; ++w, p += 2 * NB) {
+        s[w] = 0.0;
+        e[w] = 0;
+        bool scaled = false;
+        for (int i = 0; i < NB; ++i) {
+            s[w] += p[i];
+            if constexpr (sizeof(T) == 8) scaled = scaled || p[i] < 0.0;
+        }
+        if (scaled) {
+            s[w] = 0.0;
+            e[w] = -1000;                             // the largest of the blocks that are not zero
+            for (int i = 0; i < NB; ++i)
+                if (p[i] != 0.0) e[w] = max(e[w], p[i] < 0.0 ? int(p[NB + i]) : 0);
+            for (int i = 0; i < NB; ++i)
+                s[w] += ldexp(fabs(p[i]), 2 * ((p[i] < 0.0 ? int(p[NB + i]) : 0) - e[w]));
+        }
     }
-    if (!(f > 0.0 && g > 0.0 && f < 1e300 && g < 1e300)) return T(1);
-    int e = (ilogb(f) - ilogb(g)) / 2;
-    constexpr int most = sizeof(T) == 8 ? 400 : 40;
-    e = e > most ? most : (e < -most ? -most : e);
-    return T(ldexp(1.0, e));
+    BiScale c{0, 0, false};
+    if (!(s[0] < 1e300 && s[1] < 1e300)) return c;
+    c.zero = s[0] == 0.0 || s[1] == 0.0;
+    // log2 |F|^2, |G|^2, rounded down
+    const int lf = s[0] > 0.0 ? ilogb(s[0]) + 2 * e[0] : 0;
+    const int lg = s[1] > 0.0 ? ilogb(s[1]) + 2 * e[1] : 0;
+    constexpr int most = sizeof(T) == 8 ? 1000 : 120;      // times a phase: still normal
+    auto clamp = [](int x) { return x > most ? most : (x < -most ? -most : x); };
+    c.f = clamp(-(lf / 2));
+    c.g = clamp((lf - lg) / 2 - lf / 2);
+    return c;
 }
 
 constexpr int kBiXWG = 128, kBiXD = 8;             // threads; products staged at a time
@@ -146,24 +207,25 @@ struct BiNyq {
         const cplx<T>* e2 = e1 + 3 * N;
         // the (row, column) axes of the plane; s is its fixed axis
         const int ra = s == 0 ? 1 : 0, ca = s == 2 ? 1 : 2;
-        auto kap = [&](const cplx<T>* e, int a, int b) {
+        auto kap = [&](const cplx<T>* e, int a, int b, T hs) {   // 2 hs kap
             const cplx<T> E = e[s * N + H], ea = e[ra * N + a], eb = e[ca * N + b];
             const cplx<T> p = ea * eb;
             const cplx<T> pt = (a == H ? conj(ea) : ea) * (b == H ? conj(eb) : eb);
             const cplx<T> v = E * p - conj(E) * pt;
-            return mk(T(0.5) * v.y, T(-0.5) * v.x);               // v / (2i)
+            return mk(hs * v.y, -hs * v.x);                       // 2 hs v / (2i)
         };
         cplx<T>* P = L + sl * N * (N + 1);
         cplx<T> x[H], o[H];
         if (live) {
-            const T sg = bi_scale<T, N>(norm, int(t));
+            const BiScale sc = bi_scale<T, N>(norm, int(t));
+            const T hf = T(ldexp(0.5, sc.f)), hg = T(ldexp(0.5, sc.g));
             sfor<0, H>([&](auto K) {
                 const int c = 2 * int(K) + h;                     // column index of this load
                 const int l1 = s == 0 ? H : r, l2 = s == 0 ? r : (s == 1 ? H : c);
                 const int l3 = s == 2 ? H : c;
                 const bool zero = (s == 1 && r == H) || (s == 2 && (r == H || c == H));
                 const size_t at = size_t(l1) * NN + Gm::pen(l2, l3);
-                const cplx<T> a = kap(e1, r, c) * Ff[at], b = kap(e2, r, c) * (sg * Fg[at]);
+                const cplx<T> a = kap(e1, r, c, hf) * Ff[at], b = kap(e2, r, c, hg) * Fg[at];
                 x[K] = zero ? mk(T(0), T(0)) : mk(a.x - b.y, a.y + b.x);
             });
             pair_dft_dit<T, N, +1>(x, o, h);
@@ -183,7 +245,7 @@ struct BiNyq {
 };
 
 // Work-groups below nxb: Y[t][d][x][p] = sum_l1 e^{2 pi i l1 x / N}
-// (e1 F + i e2 G)(l1, p), a lane pair per pencil holds its F and G in
+// (2^f e1 F + i 2^g e2 G)(l1, p), a lane pair per pencil holds its F and G in
 // registers over a group of products.  The others: the Nyquist planes.
 template <typename T, int N>
 __global__ void __launch_bounds__(kBiXWG, 2)
@@ -194,6 +256,7 @@ k_bi_x(const cplx<T>* __restrict__ F, const cplx<T>* __restrict__ phase,
     using Ny = BiNyq<T, N>;
     constexpr int H = Gm::H, NN = Gm::NN, n = Gm::n, EX = kBiXD * 2 * N;
     __shared__ cplx<T> sh[EX > Ny::LDS ? EX : Ny::LDS];
+    __shared__ T scl[2];                              // 2^f, 2^g
     if (int(blockIdx.x) >= nxb) {
         Ny::run(sh, int(blockIdx.x) - nxb, nslot, F, phase, norm, ND, dstride,
                 nyq);
@@ -212,14 +275,19 @@ k_bi_x(const cplx<T>* __restrict__ F, const cplx<T>* __restrict__ phase,
     cplx<T> f[H], gg[H];
     const cplx<T>* Ff = F + size_t(t) * 2 * n + size_t(h) * NN + p;
     sfor<0, H>([&](auto K) { f[K] = Ff[size_t(2 * int(K)) * NN]; });
-    const T sg = bi_scale<T, N>(norm, t);
-    sfor<0, H>([&](auto K) { gg[K] = sg * Ff[n + size_t(2 * int(K)) * NN]; });
+    sfor<0, H>([&](auto K) { gg[K] = Ff[n + size_t(2 * int(K)) * NN]; });
+    if (threadIdx.x == 0) {                           // in LDS: registers are short here
+        const BiScale sc = bi_scale<T, N>(norm, t);
+        scl[0] = T(ldexp(1.0, sc.f));
+        scl[1] = T(ldexp(1.0, sc.g));
+    }
     for (int db = d0; db < d1; db += kBiXD) {
         const int nd = d1 - db < kBiXD ? d1 - db : kBiXD;
         __syncthreads();
         for (int i = threadIdx.x; i < nd * 2 * N; i += kBiXWG) {
             const int dd = i / (2 * N), k = i - dd * 2 * N, sd = k / N;
-            ex[dd][sd][k - sd * N] = phase[(size_t(db + dd) * dstride * 2 + sd) * 3 * N + k - sd * N];
+            ex[dd][sd][k - sd * N] = scl[sd] *
+                phase[(size_t(db + dd) * dstride * 2 + sd) * 3 * N + k - sd * N];
         }
         __syncthreads();
         for (int dd = 0; dd < nd; ++dd) {
@@ -470,8 +538,11 @@ k_bi_pen(const cplx<T>* __restrict__ Gp, int XG, int QB, const cplx<T>* __restri
     if (wave == 0) {
         for (int w = 0; w < NW - 1; ++w)
             sfor<0, H>([&](auto M) { g[M] = g[M] + sh[(w * H + int(M)) * 64 + lane]; });
-        const T inv = T(1) / bi_scale<T, N>(norm, t);
-        sfor<0, H>([&](auto M) { g[M] = inv * g[M]; });
+        const BiScale sc = bi_scale<T, N>(norm, t);
+        const int back = -(sc.f + sc.g);
+        sfor<0, H>([&](auto M) {
+            g[M] = sc.zero ? T(0) * g[M] : mk(T(ldexp(g[M].x, back)), T(ldexp(g[M].y, back)));
+        });
     } else {
         const cplx<T>* Fg = F + (size_t(t) * 2 + 1) * n + size_t(h) * NN + (k3 <= H ? q : 0);
         sfor<0, H>([&](auto M) {

@@ -293,7 +293,7 @@ extern "C" int dgfs_bi_collision_plan_create(int N, int M, int Nrho, double L, c
         hipMalloc(&pl->ctab, sizes.ctab * cs) != hipSuccess ||
         hipMalloc(&pl->Fhat, lchunk * 2 * n * cs) != hipSuccess ||
         hipMalloc(&pl->Iw, lchunk * 2 * n * cs) != hipSuccess ||
-        hipMalloc(&pl->norm, lchunk * 2 * dgfs::bi_norm_blocks(N) * sizeof(double)) != hipSuccess ||
+        hipMalloc(&pl->norm, lchunk * 4 * dgfs::bi_norm_blocks(N) * sizeof(double)) != hipSuccess ||
         (sizes.acc && hipMalloc(&pl->acc, chunk * sizes.acc * cs) != hipSuccess) ||
         (pl->nspec && hipMalloc(&pl->spec, pl->nspec * sizes.spec * cs) != hipSuccess) ||
         hipMalloc(&pl->H, size_t(ntask_max) * 2 * n * cs) != hipSuccess ||

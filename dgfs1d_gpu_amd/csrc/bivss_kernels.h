@@ -215,7 +215,7 @@ struct BiPlan {
     void* spec = nullptr;   // streaming: [chunk][Nrho*M][XS][NPH] cplx<T>
     void* acc = nullptr;    // [chunk][Nrho*M][n] cplx<T>
     void* H = nullptr;      // [ntask_max][2][n] cplx<T>: loss, gain
-    void* norm = nullptr;   // streaming: [like_chunk][2][bi_norm_blocks] FP64
+    void* norm = nullptr;   // streaming: [like_chunk][2][2][bi_norm_blocks] FP64
     void* Gp = nullptr;     // [chunk][groups][n] cplx<T>  partial G^; streaming: [ngrp][H][NPT][2]
 };
 

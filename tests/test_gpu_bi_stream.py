@@ -147,6 +147,88 @@ def test_trace_species(cuda, ratio):
     assert err < 3e-5
 
 
+# (streaming) plans of one pair, with the task capacity that takes them over the
+# line between the forms at N = 20, 24
+ABSENT = [(20, 'F64'), (20, 'F32'), (24, 'F64'), (24, 'F32'), (32, 'F64'), (32, 'F32'),
+          (48, 'F32')]
+
+
+def _plan(cuda, N, dtype, p, q, Nrho=3, M=6):
+    from dgfs1d_gpu_amd import _lib
+    from dgfs1d_gpu_amd.collision import BiCollisionPlan
+    vm = _mesh(N, M, Nrho)
+    m = vm.masses
+    sz, szpre = load_design('womersley', M), load_design('womersley', 32)
+    plan = BiCollisionPlan(N, M, Nrho, vm.L, vm.qz, vm.qw, sz, vm.sw, szpre, m[p], m[q], 1.36,
+                           0.8, 0.41, getattr(_lib, dtype), 80, device=cuda)
+    pre = OB.BiPrecomp(N, vm.L, vm.qz, vm.qw, sz, vm.sw, szpre, m[p], m[q], 1.36, 0.8)
+    return vm, plan, pre
+
+
+@pytest.mark.parametrize('N,dtype', ABSENT)
+def test_absent_species(cuda, N, dtype):
+    """Where a species is absent the pair's term is exactly zero, beside nodes
+    that hold both; where the present side is not finite the term is not
+    either.  The like-species form too."""
+    import torch
+    td = torch.float64 if dtype == 'F64' else torch.float32
+    tasks = [(s, [(s, 1.0)], [(s, 1.0)]) for s in range(4)]
+    for p, q in ((0, 1), (1, 1)):
+        vm, plan, _ = _plan(cuda, N, dtype, p, q)
+        u = _fields(vm, 2, 2, 11)
+        plan.set_tasks(2, 2, tasks)
+        full = [torch.tensor(u[s], dtype=td, device=cuda) for s in (p, q)]
+        if p == q:
+            full[1] = full[0]
+
+        def call(f, g):
+            Q = torch.full((4, N ** 3), 0.25, dtype=td, device=cuda)
+            plan(f, g, Q)
+            return Q
+
+        base = call(*full)
+        f, g = full[0].clone(), full[1].clone()
+        f[1], g[2] = 0.0, 0.0
+        if p == q:
+            g[1] = f[2] = 0.0
+        f[3], g[3] = 0.0, 0.0
+        got = call(f, f if p == q else g)
+        assert torch.equal(got[0], base[0]) and not torch.equal(base[0], torch.full_like(base[0], 0.25))
+        for s in (1, 2, 3):
+            assert torch.equal(got[s], torch.full_like(got[s], 0.25)), (p, q, s)
+        if p != q:
+            g[1] = float('nan')
+            f[2] = float('inf')
+            bad = call(f, g)
+            assert torch.equal(bad[0], base[0])
+            assert bool(bad[1].isnan().all()) and bool(bad[2].isnan().all())
+        plan.close()
+
+
+@pytest.mark.parametrize('N,dtype,a,b', [
+    (32, 'F32', 1e-18, 1.0), (24, 'F32', 1e18, 1.0), (20, 'F32', 1e-30, 1e25),
+    (32, 'F32', 1e20, 1e-25), (20, 'F64', 1e-200, 1e150), (24, 'F64', 1e160, 1e-170),
+    (32, 'F64', 1e-40, 1.0)])
+def test_density_range(cuda, N, dtype, a, b):
+    """Densities from end to end of the type's range: the sides of a shared
+    transform keep the precision that each has alone.  The oracle is bilinear in
+    the densities, so it is taken at 1 and scaled."""
+    import torch
+    td = torch.float64 if dtype == 'F64' else torch.float32
+    vm, plan, pre = _plan(cuda, N, dtype, 0, 1)
+    u = _fields(vm, 2, 2, 11)
+    plan.set_tasks(2, 2, [(0, [(0, 1.0)], [(1, 1.0)])])
+    up = torch.tensor(u[0] * a, dtype=td, device=cuda)
+    uq = torch.tensor(u[1] * b, dtype=td, device=cuda)
+    Q = torch.zeros_like(up)
+    plan(up, uq, Q)
+    ref = OB.q_pq(pre, u[0][0], u[1][1], 0.41)
+    err = np.abs(Q[0].double().cpu().numpy() / (a * b) - ref).max() / np.abs(ref).max()
+    plan.close()
+    print('densities', N, dtype, a, b, err, flush=True)
+    assert err < (1e-11 if dtype == 'F64' else 3e-5)
+
+
 @pytest.mark.parametrize('like', [False, True])
 def test_chunks(cuda, monkeypatch, like):
     """One and two tasks per chunk (twice that where a call shares products;

@@ -589,7 +589,8 @@ k_bi_out(const T* __restrict__ u, TaskView tv, const cplx<T>* __restrict__ Z, lo
     sfor<0, PN>([&](auto K) { s[K] = T(0); });
     const int rounds = most;
     for (int i = 0; i < rounds; ++i) {
-        const int t = ta + (i < nt ? i : nt - 1);     // a shorter slot repeats its last task
+        // a shorter slot repeats its last task, one of an empty group task 0
+        const int t = nt ? ta + (i < nt ? i : nt - 1) : 0;
         cplx<T> a[PN], o[PN];
         auto field = [&](int which) {                 // Re o = the field of column z = r
             const cplx<T>* Zp = Z + ((size_t(t) * 2 + which) * N + x) * NN;

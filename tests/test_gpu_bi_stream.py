@@ -229,6 +229,32 @@ def test_density_range(cuda, N, dtype, a, b):
     assert err < (1e-11 if dtype == 'F64' else 3e-5)
 
 
+@pytest.mark.parametrize('N,dtype', ABSENT + [(16, 'F64')])
+def test_empty_groups(cuda, N, dtype):
+    """Groups without tasks, first and last, beside others in a work-group:
+    their outputs stay, the others are those of the table without them."""
+    import torch
+    td = torch.float64 if dtype == 'F64' else torch.float32
+    vm, plan, _ = _plan(cuda, N, dtype, 0, 1)
+    u = _fields(vm, 2, 2, 11)
+    up, uq = (torch.tensor(x, dtype=td, device=cuda) for x in u)
+    t = plan.set_tasks(2, 2, [(1, [(0, 1.0)], [(1, 1.0)]), (1, [(2, 0.5)], [(3, 1.0)]),
+                              (2, [(1, 1.0)], [(0, 2.0)]), (2, [(3, 1.0)], [(3, 1.0)]),
+                              (2, [(2, 1.0)], [(2, 1.0)])])
+    ints = lambda x: torch.tensor(x, dtype=torch.int32, device=cuda)
+    assert t['gstart'].tolist() == [0, 2, 5] and t['gslice'].tolist() == [1, 2]
+    gaps = dict(t, ngroup=4, gstart=ints([0, 0, 2, 5, 5]), gslice=ints([0, 1, 2, 3]))
+    got = []
+    for table in (t, gaps):
+        Q = torch.full((4, N ** 3), 0.25, dtype=td, device=cuda)
+        plan(up, uq, Q, tasks=table)
+        got.append(Q)
+    assert torch.equal(got[0], got[1])
+    for s in (0, 3):
+        assert torch.equal(got[1][s], torch.full_like(got[1][s], 0.25))
+    plan.close()
+
+
 @pytest.mark.parametrize('like', [False, True])
 def test_chunks(cuda, monkeypatch, like):
     """One and two tasks per chunk (twice that where a call shares products;

@@ -23,6 +23,12 @@ def _bilinear_forms(tasks):
     return out
 
 
+def _form_sizes(tasks):
+    """_bilinear_forms of the magnitudes: what the rounding of a sum scales with."""
+    return _bilinear_forms([(o, [(a, abs(c)) for a, c in f], [(b, abs(c)) for b, c in g])
+                            for o, f, g in tasks])
+
+
 def _symmetric(tasks):
     """Whether the tasks of every output slice add up to a form symmetric in f
     and g, to FP64 rounding."""
@@ -91,14 +97,22 @@ PAIR_WORK = 20 << 20
 
 def pair_table(K, Ne, tasks, tdtype, device):
     """Device tables of dgfs_collide_pairs for a list of tasks, or None where the
-    tasks themselves need no more transforms.  A task costs one transform per
-    direction when every task has f = g and two otherwise; a pair (b, b) one, a
-    pair (a, b) two."""
+    tasks themselves need no more transforms, or where a product of coefficients
+    is no normal number of the type.  A task costs one transform per direction
+    when every task has f = g and two otherwise; a pair (b, b) one, a pair (a, b)
+    two."""
     import torch
+    lim = np.finfo(np.float64 if tdtype == torch.float64 else np.float32)
+    least, most = float(lim.tiny), float(lim.max)
+    if any(ca and cb and not least <= abs(ca * cb) <= most
+           for _, f, g in tasks for _, ca in f for _, cb in g):
+        return None
     out = _bilinear_forms(tasks)
-    for T in out.values():                     # what is left of exact zeros
-        most = max((abs(v) for v in T.values()), default=0.0)
-        for ab in [ab for ab, v in T.items() if abs(v) <= 1e-15 * most]:
+    size = _form_sizes(tasks)
+    if any(v > most for T in size.values() for v in T.values()):
+        return None
+    for o, T in out.items():                   # products that cancel, up to their rounding
+        for ab in [ab for ab, v in T.items() if abs(v) <= 4e-15 * size[o][ab]]:
             del T[ab]
     diag = sorted({b for T in out.values() for _, b in T})
     off = sorted({(min(ab), max(ab)) for T in out.values() for ab in T if ab[0] != ab[1]})

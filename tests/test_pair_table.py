@@ -85,6 +85,34 @@ def test_tables_without_gain_keep_their_tasks():
     assert pair_table(2, 2, [], torch.float64, 'cpu') is None
 
 
+@pytest.mark.parametrize('bad,dtype', [(float('inf'), 'float64'), (float('nan'), 'float64'),
+                                       (1e200, 'float64'), (1e30, 'float32'), (1e-30, 'float32'),
+                                       (1e-170, 'float64')])
+def test_coefficients_out_of_range_keep_their_tasks(bad, dtype):
+    """Products of coefficients that are not finite or no normal numbers of the
+    type: the tasks give what they always gave for them, no output is dropped."""
+    import torch
+    td = getattr(torch, dtype)
+    good = [(o, [(0, 1.0), (1, 0.5)], [(0, c), (1, 2.0)]) for o in range(4) for c in (1.0, 3.0)]
+    assert pair_table(4, 1, good, td, 'cpu') is not None
+    for at in range(2):
+        worse = list(good)
+        worse[5] = (2, [(at, bad)], [(0, bad)])
+        assert pair_table(4, 1, worse, td, 'cpu') is None
+
+
+def test_small_coefficients_stay():
+    """A coefficient far below its output's largest belongs to a slice that may be
+    as much larger: only products that cancel are left out."""
+    tasks = [(o, [(0, 1.0), (1, 1e-9)], [(0, c), (1, 2e-9)]) for o in range(4) for c in (1.0, 3.0)]
+    got = _forms(_check(4, 1, tasks), 4)
+    for o in range(4):
+        assert abs(got[o][1][1, 1] - 4e-18) <= 1e-32
+    zero = [(o, [(0, 1.0), (1, c)], [(0, 0.3), (1, 0.7 * c)]) for o in range(4) for c in (1.0, -1.0)]
+    p = _check(4, 1, zero)                     # (0, 1) and (1, 0) cancel
+    assert p['npair'] == p['ndiag'] == 2
+
+
 def test_symmetric_flag():
     """task_table marks exactly the tables whose outputs are symmetric in f and g."""
     import torch

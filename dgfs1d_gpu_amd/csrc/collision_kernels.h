@@ -259,6 +259,65 @@ k_nyq(const cplx<T>* __restrict__ FN, const cplx<T>* __restrict__ phase, int M, 
     });
 }
 
+// The same planes one per sign and N-thread slot, a lane per row, straight from
+// F^: for few work-groups (nyq_gathers).
+template <typename T, int N>
+__global__ void __launch_bounds__(6 * N)
+k_nyq_lane(const cplx<T>* __restrict__ Fhat, const cplx<T>* __restrict__ phase, int M, int Nrho,
+           int NW, T* __restrict__ nyq) {
+    // one 2D plane per N-thread slot: slot = 2 type + sign; thread c walks k
+    constexpr int NN = N * N, n = N * NN, PS = N * (N + 1), H = N / 2;
+    __shared__ cplx<T> L[6 * PS];
+    const int bid = blockIdx.x;
+    const int q = bid % M, p = (bid / M) % Nrho, w = (bid / (M * Nrho)) % NW;
+    const int t = bid / (M * Nrho * NW);
+    const cplx<T>* F = Fhat + (size_t(t) * 2 + w) * n;
+    const cplx<T>* ph = phase + (size_t(p) * M + q) * 3 * N;
+    const int slot = threadIdx.x / N, c = threadIdx.x - slot * N;
+    const int type = slot >> 1;
+    const bool minus = (slot & 1) != 0;
+    cplx<T>* P = L + slot * PS;
+    // loads: rows a, columns b of the plane (A: a = l2, b = l3; B: a = l1,
+    // b = l3; C: a = l1, b = l2); consecutive threads read consecutive l2
+    // where the plane has an l2 axis (A, C)
+    if (type == 0) {                       // thread c = l2, k = l3
+        const cplx<T> e0 = ph[H] * ph[N + c];
+        sfor<0, N>([&](auto K) {
+            constexpr int k = K;
+            const cplx<T> e = e0 * ph[2 * N + k];
+            P[c * (N + 1) + k] = cmul_conj_if(F[(size_t(k) * N + H) * N + c], e, minus);
+        });
+    } else if (type == 1) {                // thread c = l1, k = l3
+        const cplx<T> e0 = ph[c] * ph[N + H];
+        const bool zero = c == H;
+        sfor<0, N>([&](auto K) {
+            constexpr int k = K;
+            const cplx<T> e = e0 * ph[2 * N + k];
+            const cplx<T> v = cmul_conj_if(F[(size_t(k) * N + c) * N + H], e, minus);
+            P[c * (N + 1) + k] = zero ? mk(T(0), T(0)) : v;
+        });
+    } else {                               // thread c = l2, k = l1
+        const cplx<T> e0 = ph[N + c] * ph[2 * N + H];
+        sfor<0, N>([&](auto K) {
+            constexpr int k = K;
+            const cplx<T> e = ph[k] * e0;
+            const cplx<T> v = cmul_conj_if(F[(size_t(H) * N + k) * N + c], e, minus);
+            P[k * (N + 1) + c] = (k == H || c == H) ? mk(T(0), T(0)) : v;
+        });
+    }
+    __syncthreads();
+    lds_fft_row<T, N, +1>(P, c);          // over b for row c
+    __syncthreads();
+    lds_fft_col<T, N, +1>(P, c);          // over a for column c
+    __syncthreads();
+    // stores (coalesced): A[y][z] = P[y][z]; B[z][x] = P[x][z]; C[y][x] = P[x][y]
+    T* dst = nyq + ((((size_t(t) * NW + w) * Nrho + p) * M + q) * 6 + slot) * NN;
+    sfor<0, N>([&](auto K) {
+        constexpr int k = K;
+        dst[k * N + c] = (type == 0) ? P[k * (N + 1) + c].y : P[c * (N + 1) + k].y;
+    });
+}
+
 // LDS image of one (which)'s Nyquist data for residue r, row pitch BP
 template <int N, int S>
 struct NyLayout {
@@ -1021,6 +1080,22 @@ inline void timing_mark(CollisionPlan* pl, int stage, hipStream_t st) {
 
 // -------------------------------------------------------------- launch
 
+// Which form of the Nyquist planes a call of so many (function, p, q) takes:
+// k_nyq's transforms are half as many, but each is a longer chain on lane
+// pairs, and gathering its planes lengthens k_fwd_line's.  us of a whole call,
+// k_nyq_lane / k_nyq, by count:
+//   FP32 N = 20: 288 123.1/123.3, 576 101.1/100.5, 1152 131.6/129.2
+//   FP32 N = 24: 144 89.4/89.6, 576 120.1/119.1, 1152 166.0/161.9
+//   FP32 N = 32: 90 64.9/67.1, 432 118.5/119.8, 576 123.9/123.0, 1152 157.2/152.4
+//   FP32 N = 48: 90 384.9/385.9, 144 596.0/596.0, 288 762.5/759.6
+//   FP64 N = 12: 288 77.8/77.8, 768 84.7/84.0;  N = 16: 432 57.8/58.3
+//   FP64 N = 20: 90 90.6/90.9, 288 151.4/149.8;  N = 24: 90 112.5/112.7, 288 196.3/195.0
+//   FP64 N = 32: 30 130.0/135.3, 144 175.6/178.0, 288 235.6/232.0, 1152 384.5/368.5
+template <typename T, int N>
+constexpr bool nyq_gathers(long groups) {
+    return groups >= (N >= 48 || (sizeof(T) == 8 && N >= 20) ? 256 : 512);
+}
+
 template <typename T, int N>
 struct Impl {
     static constexpr int S1 = pick_split_gain<T, N, 1>();   // gain residue split, f = g
@@ -1054,9 +1129,11 @@ struct Impl {
         const int nfg = fg_same ? 1 : 2;
         constexpr long NN = long(N) * N;
         timing_mark(pl, 0, st);
-        if (int rc = forward(pl, u, ug, tv, ntask, nfg, dev, (cplx<T>*)pl->Fhat, st)) return rc;
+        cplx<T>* F = (cplx<T>*)pl->Fhat;
+        const bool gather = nyq_gathers<T, N>(long(ntask) * nfg * pl->Nrho * pl->M);
+        if (int rc = forward(pl, u, ug, tv, ntask, nfg, dev, F, gather, st)) return rc;
         timing_mark(pl, 1, st);
-        if (int rc = nyquist(pl, 0, ntask, nfg, st)) return rc;
+        if (int rc = nyquist(pl, 0, ntask, nfg, F, gather, st)) return rc;
         timing_mark(pl, 2, st);
         int S = S1;
         if (dev) {
@@ -1146,12 +1223,20 @@ struct Impl {
         return 0;
     }
 
-    // Nyquist planes of nw functions of those tasks
-    static int nyquist(CollisionPlan* pl, int t0, int cnt, int nw, hipStream_t st) {
-        hipLaunchKernelGGL((k_nyq<T, N>), dim3(cnt * nw * pl->Nrho * pl->M), dim3(6 * N), 0, st,
-                           (const cplx<T>*)pl->FN + size_t(t0) * 2 * 3 * N * N,
-                           (const cplx<T>*)pl->phase, pl->M, pl->Nrho, nw,
-                           (T*)pl->nyq + size_t(t0) * 2 * pl->Nrho * pl->M * 6 * N * N);
+    // Nyquist planes of nw functions of those tasks, from the F^ that forward
+    // wrote to F (gather: from FN)
+    static int nyquist(CollisionPlan* pl, int t0, int cnt, int nw, const cplx<T>* F, bool gather,
+                       hipStream_t st) {
+        const dim3 nb(cnt * nw * pl->Nrho * pl->M), wg(6 * N);
+        const cplx<T>* ph = (const cplx<T>*)pl->phase;
+        T* ny = (T*)pl->nyq + size_t(t0) * 2 * pl->Nrho * pl->M * 6 * N * N;
+        if (gather)
+            hipLaunchKernelGGL((k_nyq<T, N>), nb, wg, 0, st,
+                               (const cplx<T>*)pl->FN + size_t(t0) * 2 * 3 * N * N, ph, pl->M,
+                               pl->Nrho, nw, ny);
+        else
+            hipLaunchKernelGGL((k_nyq_lane<T, N>), nb, wg, 0, st, F + size_t(t0) * 2 * pl->n, ph,
+                               pl->M, pl->Nrho, nw, ny);
         DGFS_HIP_CHECK(hipGetLastError());
         return 0;
     }
@@ -1161,11 +1246,13 @@ struct Impl {
                             int ndiag, PairOutput po, int nout, hipStream_t st) {
         const int noff = npair - ndiag;
         timing_mark(pl, 0, st);
-        if (int rc = forward(pl, u, u, tv, npair, 2, false, (cplx<T>*)pl->Fhat, st)) return rc;
+        cplx<T>* F = (cplx<T>*)pl->Fhat;
+        const bool gather = nyq_gathers<T, N>(long(ndiag + 2 * noff) * pl->Nrho * pl->M);
+        if (int rc = forward(pl, u, u, tv, npair, 2, false, F, gather, st)) return rc;
         timing_mark(pl, 1, st);
-        if (int rc = nyquist(pl, 0, ndiag, 1, st)) return rc;
+        if (int rc = nyquist(pl, 0, ndiag, 1, F, gather, st)) return rc;
         if (noff)
-            if (int rc = nyquist(pl, ndiag, noff, 2, st)) return rc;
+            if (int rc = nyquist(pl, ndiag, noff, 2, F, gather, st)) return rc;
         timing_mark(pl, 2, st);
         int Sd = 1, So = 1;
         if (int rc = gain(pl, 0, ndiag, 1, &Sd, st)) return rc;
@@ -1186,10 +1273,11 @@ struct Impl {
         return 0;
     }
 
-    // F^ of every task into dst ([t][2][n], nfg functions per task); dev: the
-    // single function h = f - f0 (u = f, ug = f0)
+    // F^ of every task into dst ([t][2][n], nfg functions per task), with gather
+    // its Nyquist planes into FN; dev: the single function h = f - f0 (u = f,
+    // ug = f0)
     static int forward(CollisionPlan* pl, const void* u, const void* ug, TaskView tv, int ntask,
-                       int nfg, bool dev, cplx<T>* dst, hipStream_t st) {
+                       int nfg, bool dev, cplx<T>* dst, bool gather, hipStream_t st) {
         constexpr long NN = long(N) * N;
         const long npl = long(ntask) * nfg * N;
         constexpr int FP = fwd_planes_per_wg(N);
@@ -1203,7 +1291,7 @@ struct Impl {
         DGFS_HIP_CHECK(hipGetLastError());
         const long nli = long(ntask) * nfg * NN;
         hipLaunchKernelGGL((k_fwd_line<T, N>), dim3((nli + 255) / 256), dim3(256), 0, st, nli,
-                           nfg, (const cplx<T>*)pl->Iw, dst, (cplx<T>*)pl->FN);
+                           nfg, (const cplx<T>*)pl->Iw, dst, gather ? (cplx<T>*)pl->FN : nullptr);
         DGFS_HIP_CHECK(hipGetLastError());
         return 0;
     }
@@ -1212,8 +1300,10 @@ struct Impl {
     // (task, p, q) into the plan's reference buffers
     static int reference_set(CollisionPlan* pl, const void* u0, TaskView tv, int ntask,
                              hipStream_t st) {
-        if (int rc = forward(pl, u0, u0, tv, ntask, 1, false, (cplx<T>*)pl->Fhat0, st)) return rc;
-        if (int rc = nyquist(pl, 0, ntask, 1, st)) return rc;
+        cplx<T>* F = (cplx<T>*)pl->Fhat0;
+        const bool gather = nyq_gathers<T, N>(long(ntask) * pl->Nrho * pl->M);
+        if (int rc = forward(pl, u0, u0, tv, ntask, 1, false, F, gather, st)) return rc;
+        if (int rc = nyquist(pl, 0, ntask, 1, F, gather, st)) return rc;
         const int nb = ntask * pl->Nrho * S1 * pl->QG;
         // the store pass lays the pairs out for the delta kernel that reads them
         if constexpr (kPair)

@@ -328,21 +328,19 @@ struct NyLayout {
     static constexpr int SIZE = C + 2 * N * BP;
 };
 
-// Staging of a (task, p, q)'s Nyquist data for residue r by NT threads: item
-// i = A+- [y][j], B+- [j][x], C+- [y][x] of the NW functions in turn.  load()
+// Staging of a (task, p, q)'s Nyquist data for residue r by NT threads: items
+// A+- [y][j], B+- [j][x], C+- [y][x] of the NW functions in turn.  load()
 // issues all of a thread's loads, store() puts them into the LDS image, so
 // that one memory latency and not one per item is paid (and none where the
-// loads are issued a pass ahead).
+// loads are issued a pass ahead); copy<D>() keeps D items in flight at a time.
 template <typename T, int N, int S, int NW, int NT>
 struct NyStage {
     using NL = NyLayout<N, S>;
     static constexpr int NS = N / S, NN = N * N, BP = NL::BP;
     static constexpr int PER = 4 * N * NS + 2 * NN, ITEMS = NW * PER, K = (ITEMS + NT - 1) / NT;
     T v[K];
-    // src: this (t, w = 0, p, q)'s planes; wstride: from one function's to the next
-    static DGFS_DEV T get(int i, const T* src, size_t wstride, int r) {
-        const int w = NW == 1 ? 0 : i / PER, k = NW == 1 ? i : i - w * PER;
-        const T* s = src + w * wstride;
+    // item k of one function: s its planes, d its LDS image
+    static DGFS_DEV T one(int k, const T* s, int r) {
         if (k < 2 * N * NS) {                            // A: e = y NS + j
             const int sg = k / (N * NS), e = k - sg * N * NS;
             return s[sg * NN + (e / NS) * N + S * (e % NS) + r];
@@ -353,9 +351,7 @@ struct NyStage {
         }
         return s[4 * NN + k - 4 * N * NS];               // C: e = y N + x
     }
-    static DGFS_DEV void put(int i, T x, T* Ny) {
-        const int w = NW == 1 ? 0 : i / PER, k = NW == 1 ? i : i - w * PER;
-        T* d = Ny + w * NL::SIZE;
+    static DGFS_DEV void set(int k, T x, T* d) {
         if (k < 2 * N * NS) {
             d[NL::A + k] = x;
         } else if (k < 4 * N * NS) {
@@ -365,6 +361,15 @@ struct NyStage {
             const int k2 = k - 4 * N * NS, sg = k2 / NN, e = k2 - sg * NN;
             d[NL::C + sg * N * BP + (e / N) * BP + e % N] = x;
         }
+    }
+    // src: this (t, w = 0, p, q)'s planes; wstride: from one function's to the next
+    static DGFS_DEV T get(int i, const T* src, size_t wstride, int r) {
+        const int w = NW == 1 ? 0 : i / PER;
+        return one(i - w * PER, src + w * wstride, r);
+    }
+    static DGFS_DEV void put(int i, T x, T* Ny) {
+        const int w = NW == 1 ? 0 : i / PER;
+        set(i - w * PER, x, Ny + w * NL::SIZE);
     }
     DGFS_DEV void load(const T* src, size_t wstride, int r) {
         sfor<0, K>([&](auto Ki) {
@@ -378,7 +383,57 @@ struct NyStage {
             if (i < ITEMS) put(i, v[Ki], Ny);
         });
     }
+    template <int D>
+    static DGFS_DEV void copy(const T* src, size_t wstride, int r, T* Ny) {
+        if constexpr (D == 1) {
+            sfor<0, NW>([&](auto W) {
+                for (int k = threadIdx.x; k < PER; k += NT)
+                    set(k, one(k, src + int(W) * wstride, r), Ny + int(W) * NL::SIZE);
+            });
+        } else {
+            for (int i0 = threadIdx.x; i0 < ITEMS; i0 += D * NT) {
+                T x[D];
+                sfor<0, D>([&](auto Ki) {
+                    if (i0 + int(Ki) * NT < ITEMS) x[Ki] = get(i0 + int(Ki) * NT, src, wstride, r);
+                });
+                sfor<0, D>([&](auto Ki) {
+                    if (i0 + int(Ki) * NT < ITEMS) put(i0 + int(Ki) * NT, x[Ki], Ny);
+                });
+            }
+        }
+    }
 };
+
+// Waves per SIMD that k_gain is held to: with the staging's loads in flight the
+// compiler takes some registers more than these allow and halves the waves in
+// flight.  Without, with: FP64 N = 12, f != g, 18432 (function, p, q) 366/244 us;
+// the twofold split (PAD = 0) of FP64 N = 24, 2304 of them, 602/413 us, and of
+// FP32 N = 48, 288 of them, 1657/1031 us.
+template <typename T, int N, int S, int NW, int PAD>
+constexpr int gain_waves() {
+    if (sizeof(T) == 8 && N == 12) return NW == 2 ? 2 : 3;
+    if (PAD == 0 && (N == 48 || (sizeof(T) == 8 && N == 24))) return 2;
+    return 1;
+}
+
+// Items in flight per thread in k_gain's staging, 0: all of them, which wins
+// but where it takes the registers of the transforms (spills).  few: fewer
+// than kNyqFew (function, p, q), where one work-group per CU or less runs and
+// the spills are not hidden.  us for all / for the number here, by count:
+//   FP64 N = 20, f = g: 576 138/135, 2304 236/231
+//   N = 24, f = g: FP32 576 119.5/116.0, 1152 162.1/161.3, 2304 190.0/190.7,
+//     15360 729/782; FP64 90 112.7/110.4, 1152 220.3/219.9, 15360 1948/1969
+//   N = 24, f != g: FP32 240 118.0/115.7, 18432 928/927; FP64 240 153.5/150.4,
+//     18432 2074/1997
+constexpr long kNyqFew = 1024;
+template <typename T, int N, int NW, int PAD>
+constexpr int nyq_in_flight(bool few) {
+    if (PAD == 0) return 0;
+    if (sizeof(T) == 8 && N == 20 && NW == 1) return 1;
+    if (N == 24 && NW == 1) return few ? (sizeof(T) == 4 ? 1 : 4) : 0;
+    if (N == 24) return sizeof(T) == 4 ? 4 : 8;
+    return 0;
+}
 
 template <typename T, int N, int S>
 constexpr int gain_lds_bytes(int NW) {
@@ -465,8 +520,9 @@ enum GainMode { kGainAccumulate = 0, kGainStore = 1, kGainDelta = 2 };
 //   ucache[t][p][q][x][r][P] (P = this thread's pencil) instead.
 // MODE kGainDelta (NW = 1, F^ = h^): acc = sum_q u+h (u-h + u-f0) + u-h u+f0
 //   with u+-_f0 read from ucache.
-template <typename T, int N, int S, int NW, int MODE = kGainAccumulate, int PAD = 1>
-__global__ void __launch_bounds__(round64(N * (N / S)))
+// D: items in flight of the staging (nyq_in_flight).
+template <typename T, int N, int S, int NW, int MODE, int PAD, int D>
+__global__ void __launch_bounds__(round64(N * (N / S)), (gain_waves<T, N, S, NW, PAD>()))
 k_gain(const cplx<T>* __restrict__ Fhat, const cplx<T>* __restrict__ phase,
        const T* __restrict__ nyq, int M, int Nrho, int QG, cplx<T>* __restrict__ acc_out,
        UPair<T>* __restrict__ ucache, int remap) {
@@ -507,16 +563,11 @@ k_gain(const cplx<T>* __restrict__ Fhat, const cplx<T>* __restrict__ phase,
                 [&] {
                     if constexpr (wv != 0) return;
                     // stage this q's Nyquist imaginary parts for residue r
-                    // FP64 grids whose N^2 lanes do not fill their waves: item by
-                    // item (all of a thread's items in flight 81 against 76 us at
-                    // N = 12, 241 against 239 at N = 20; elsewhere they win: FP64
-                    // N = 16 88/95, N = 24 337/352, FP32 N = 20 147/157 us)
                     using St = NyStage<T, N, S, NW, E::NT>;
                     const T* src = nyq + ((size_t(t) * NW * Nrho + p) * M + q) * 6 * NN;
                     const size_t ws = size_t(Nrho) * M * 6 * NN;
-                    if constexpr (sizeof(T) == 8 && N % 8 != 0) {
-                        for (int i = threadIdx.x; i < St::ITEMS; i += E::NT)
-                            St::put(i, St::get(i, src, ws, r), Ny);
+                    if constexpr (D) {
+                        St::template copy<D>(src, ws, r, Ny);
                     } else {
                         St st;
                         st.load(src, ws, r);
@@ -1137,19 +1188,16 @@ struct Impl {
         timing_mark(pl, 2, st);
         int S = S1;
         if (dev) {
-            const int nb = ntask * pl->Nrho * S1 * pl->QG;
             if constexpr (kPair)
-                hipLaunchKernelGGL((k_gain_pair<T, N, S1, kGainDelta>), dim3(nb),
+                hipLaunchKernelGGL((k_gain_pair<T, N, S1, kGainDelta>),
+                                   dim3(ntask * pl->Nrho * S1 * pl->QG),
                                    dim3(2 * N * (N / S1)), 0, st, (const cplx<T>*)pl->Fhat,
                                    (const cplx<T>*)pl->phase, (const cplx<T>*)pl->phz,
                                    (const T*)pl->nyq, pl->M, pl->Nrho, pl->QG, (cplx<T>*)pl->acc,
                                    (UPair<T>*)pl->ucache, pl->gain_remap);
             else
-                hipLaunchKernelGGL((k_gain<T, N, S1, 1, kGainDelta>), dim3(nb),
-                                   dim3(round64(N * (N / S1))), 0, st, (const cplx<T>*)pl->Fhat,
-                                   (const cplx<T>*)pl->phase, (const T*)pl->nyq, pl->M, pl->Nrho,
-                                   pl->QG, (cplx<T>*)pl->acc, (UPair<T>*)pl->ucache,
-                                   pl->gain_remap);
+                run_gain<S1, 1, kGainDelta>(pl, ntask, (const cplx<T>*)pl->Fhat,
+                                            (const T*)pl->nyq, (cplx<T>*)pl->acc, st);
             DGFS_HIP_CHECK(hipGetLastError());
         } else if (int rc = gain(pl, 0, ntask, fg_same, &S, st)) {
             return rc;
@@ -1186,30 +1234,43 @@ struct Impl {
         const bool alt = fg_same && pl->gain_smul == 2 && S1x != S1;
         const bool pair = fg_same && !alt && (kPair || kPair64);
         *S = alt ? S1x : (pair ? SP : (fg_same ? S1 : S2));
-        const dim3 nb(cnt * pl->Nrho * *S * pl->QG);
-        const int rm = pl->gain_remap, M = pl->M, Nrho = pl->Nrho, QG = pl->QG;
         const cplx<T>* F = (const cplx<T>*)pl->Fhat + size_t(t0) * 2 * pl->n;
-        const cplx<T>* ph = (const cplx<T>*)pl->phase;
-        const T* ny = (const T*)pl->nyq + size_t(t0) * 2 * Nrho * M * 6 * N * N;
-        cplx<T>* acc = (cplx<T>*)pl->acc + size_t(t0) * Nrho * QG * pl->n;
+        const T* ny = (const T*)pl->nyq + size_t(t0) * 2 * pl->Nrho * pl->M * 6 * N * N;
+        cplx<T>* acc = (cplx<T>*)pl->acc + size_t(t0) * pl->Nrho * pl->QG * pl->n;
         if (pair) {
             if constexpr (kPair || kPair64)
-                hipLaunchKernelGGL((k_gain_pair<T, N, SP, kGainAccumulate, PADP>), nb,
-                                   dim3(2 * N * (N / SP)), 0, st, F, ph, (const cplx<T>*)pl->phz,
-                                   ny, M, Nrho, QG, acc, (UPair<T>*)nullptr, rm);
+                hipLaunchKernelGGL((k_gain_pair<T, N, SP, kGainAccumulate, PADP>),
+                                   dim3(cnt * pl->Nrho * SP * pl->QG), dim3(2 * N * (N / SP)), 0,
+                                   st, F, (const cplx<T>*)pl->phase, (const cplx<T>*)pl->phz, ny,
+                                   pl->M, pl->Nrho, pl->QG, acc, (UPair<T>*)nullptr,
+                                   pl->gain_remap);
         } else if (alt) {
-            hipLaunchKernelGGL((k_gain<T, N, S1x, 1, kGainAccumulate, 0>), nb,
-                               dim3(round64(N * (N / S1x))), 0, st, F, ph, ny, M, Nrho, QG, acc,
-                               (UPair<T>*)nullptr, rm);
+            run_gain<S1x, 1, kGainAccumulate, 0>(pl, cnt, F, ny, acc, st);
         } else if (fg_same) {
-            hipLaunchKernelGGL((k_gain<T, N, S1, 1>), nb, dim3(round64(N * (N / S1))), 0, st, F,
-                               ph, ny, M, Nrho, QG, acc, (UPair<T>*)nullptr, rm);
+            run_gain<S1, 1, kGainAccumulate>(pl, cnt, F, ny, acc, st);
         } else {
-            hipLaunchKernelGGL((k_gain<T, N, S2, 2>), nb, dim3(round64(N * (N / S2))), 0, st, F,
-                               ph, ny, M, Nrho, QG, acc, (UPair<T>*)nullptr, rm);
+            run_gain<S2, 2, kGainAccumulate>(pl, cnt, F, ny, acc, st);
         }
         DGFS_HIP_CHECK(hipGetLastError());
         return 0;
+    }
+
+    // k_gain for cnt tasks
+    template <int S, int NW, int MODE, int PAD = 1>
+    static void run_gain(CollisionPlan* pl, int cnt, const cplx<T>* F, const T* ny, cplx<T>* acc,
+                         hipStream_t st) {
+        auto go = [&](auto D) {
+            hipLaunchKernelGGL((k_gain<T, N, S, NW, MODE, PAD, int(D)>),
+                               dim3(cnt * pl->Nrho * S * pl->QG), dim3(round64(N * (N / S))), 0,
+                               st, F, (const cplx<T>*)pl->phase, ny, pl->M, pl->Nrho, pl->QG, acc,
+                               MODE == kGainAccumulate ? (UPair<T>*)nullptr
+                                                       : (UPair<T>*)pl->ucache,
+                               pl->gain_remap);
+        };
+        if (long(cnt) * NW * pl->Nrho * pl->M < kNyqFew)
+            go(std::integral_constant<int, nyq_in_flight<T, N, NW, PAD>(true)>{});
+        else
+            go(std::integral_constant<int, nyq_in_flight<T, N, NW, PAD>(false)>{});
     }
 
     // the plane stage of those tasks
@@ -1304,19 +1365,17 @@ struct Impl {
         const bool gather = nyq_gathers<T, N>(long(ntask) * pl->Nrho * pl->M);
         if (int rc = forward(pl, u0, u0, tv, ntask, 1, false, F, gather, st)) return rc;
         if (int rc = nyquist(pl, 0, ntask, 1, F, gather, st)) return rc;
-        const int nb = ntask * pl->Nrho * S1 * pl->QG;
         // the store pass lays the pairs out for the delta kernel that reads them
         if constexpr (kPair)
-            hipLaunchKernelGGL((k_gain_pair<T, N, S1, kGainStore>), dim3(nb),
+            hipLaunchKernelGGL((k_gain_pair<T, N, S1, kGainStore>),
+                               dim3(ntask * pl->Nrho * S1 * pl->QG),
                                dim3(2 * N * (N / S1)), 0, st, (const cplx<T>*)pl->Fhat0,
                                (const cplx<T>*)pl->phase, (const cplx<T>*)pl->phz,
                                (const T*)pl->nyq, pl->M, pl->Nrho,
                                pl->QG, (cplx<T>*)nullptr, (UPair<T>*)pl->ucache, pl->gain_remap);
         else
-            hipLaunchKernelGGL((k_gain<T, N, S1, 1, kGainStore>), dim3(nb),
-                               dim3(round64(N * (N / S1))), 0, st, (const cplx<T>*)pl->Fhat0,
-                               (const cplx<T>*)pl->phase, (const T*)pl->nyq, pl->M, pl->Nrho,
-                               pl->QG, (cplx<T>*)nullptr, (UPair<T>*)pl->ucache, pl->gain_remap);
+            run_gain<S1, 1, kGainStore>(pl, ntask, (const cplx<T>*)pl->Fhat0, (const T*)pl->nyq,
+                                        nullptr, st);
         DGFS_HIP_CHECK(hipGetLastError());
         return 0;
     }

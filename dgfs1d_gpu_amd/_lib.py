@@ -95,6 +95,7 @@ SIGNATURES = {
                                            _d, _d, _d, _i, _i, C.POINTER(_vp)]),
     'dgfs_bi_collision_plan_destroy': (_i, [_vp]),
     'dgfs_bi_collision_plan_query': (_i, [_vp, _ip, _ip, _szp]),
+    'dgfs_bi_collision_plan_form': (_i, [_vp, _ip, _ip]),
     'dgfs_bi_collide_like': (_i, [_vp, _vp, _vp, _i, _i, _i, _vp, _vp, _vp, _i, _vp, _vp, _vp]),
     'dgfs_bi_collide': (_i, [_vp, _vp, _vp, _vp, _i, _i, _i, _vp, _vp, _vp, _i, _vp, _vp, _vp]),
     'dgfs_collision_timing_read': (_i, [_vp, _dp, _ip]),

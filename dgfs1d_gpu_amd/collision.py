@@ -343,7 +343,11 @@ class BiCollisionPlan:
         b = _lib.C.c_size_t()
         _lib.check(_lib.lib().dgfs_bi_collision_plan_query(
             self._h, _lib.C.byref(s), _lib.C.byref(ch), _lib.C.byref(b)))
-        return dict(split=s.value, chunk=ch.value, scratch_bytes=b.value)
+        st, lc = _lib.C.c_int(), _lib.C.c_int()
+        _lib.check(_lib.lib().dgfs_bi_collision_plan_form(
+            self._h, _lib.C.byref(st), _lib.C.byref(lc)))
+        return dict(split=s.value, chunk=ch.value, scratch_bytes=b.value,
+                    streaming=bool(st.value), like_chunk=lc.value)
 
     def set_tasks(self, K, Ne, tasks):
         if len(tasks) > self.ntask_max:

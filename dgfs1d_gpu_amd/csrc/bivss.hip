@@ -168,8 +168,7 @@ extern "C" int dgfs_bi_collision_plan_create(int N, int M, int Nrho, double L, c
                      N == 32 || N == 48,
                  "bi_collision_plan_create: unsupported N=%d", N);
     DGFS_REQUIRE(N != 48 || dtype == DGFS_F32,
-                 "bi_collision_plan_create: N=48 is built for DGFS_F32 only (its FP64 plane "
-                 "buffers exceed the 160 KiB LDS of a work-group)");
+                 "bi_collision_plan_create: N=48 is built for DGFS_F32 only");
     DGFS_REQUIRE(M > 0 && Nrho > 0 && Mpre > 0 && ntask_max > 0,
                  "bi_collision_plan_create: bad sizes");
     DGFS_REQUIRE(dtype == DGFS_F64 || dtype == DGFS_F32, "bi_collision_plan_create: bad dtype");
@@ -248,8 +247,7 @@ extern "C" int dgfs_bi_collision_plan_create(int N, int M, int Nrho, double L, c
     if (chunk > size_t(ntask_max)) chunk = size_t(ntask_max);
     pl->chunk = int(chunk);
     // a call that shares products takes half of them per task
-    const size_t lchunk = stream && antipodal && mp == mq
-                              ? std::min(2 * chunk, size_t(ntask_max)) : chunk;
+    const size_t lchunk = pl->shares() ? std::min(2 * chunk, size_t(ntask_max)) : chunk;
     pl->like_chunk = int(lchunk);
 
     pl->ngrp = chunk * size_t(sizes.groups);
@@ -359,6 +357,15 @@ extern "C" int dgfs_bi_collision_plan_query(dgfs_bi_collision_plan_t plan, int* 
                           pl->nspec * z.spec + pl->ngrp * z.group +
                           size_t(pl->ntask_max) * 2 * pl->n) * cs;
     }
+    return 0;
+}
+
+extern "C" int dgfs_bi_collision_plan_form(dgfs_bi_collision_plan_t plan, int* streaming,
+                                           int* like_chunk) {
+    auto* pl = static_cast<BiPlan*>(plan);
+    DGFS_REQUIRE(pl, "bi_collision_plan_form: null plan");
+    if (streaming) *streaming = pl->stream;
+    if (like_chunk) *like_chunk = pl->shares() ? pl->like_chunk : 0;
     return 0;
 }
 

@@ -202,6 +202,8 @@ struct BiPlan {
     size_t n;
     bool stream = false;    // the streaming kernels (bi_pipeline.h)
     bool antipodal = false; // the streaming form's products come in opposite pairs (2u, 2u + 1)
+    // a species with itself: the products of an opposite pair are one
+    bool shares() const { return antipodal && mp == mq; }
     size_t nspec = 0;       // planes of spec
     size_t ngrp = 0;        // partial G^ that Gp holds
     void* phase = nullptr;  // [Nrho*M][2][3][N] cplx<T>, in product order
@@ -326,7 +328,7 @@ int bi_launch(BiPlan* pl, const void* up, const void* uq, void* Q, TaskView tv, 
     constexpr long NN = long(N) * N;
     const int NXY = pl->Nrho * pl->M;
     const size_t n = pl->n;
-    like = like && pl->antipodal && pl->mp == pl->mq;
+    like = like && pl->shares();
     // even chunks: a short last one would leave the chip idle at each kernel's end
     const int most = like ? pl->like_chunk : pl->chunk;
     const int nchunk = (ntask + most - 1) / most;

@@ -179,9 +179,15 @@ int dgfs_bi_collision_plan_create(int N, int M, int Nrho, double L, const double
                                   double omega, double prefac, int dtype, int ntask_max,
                                   dgfs_bi_collision_plan_t* plan);
 int dgfs_bi_collision_plan_destroy(dgfs_bi_collision_plan_t plan);
-/* split S of the gain kernel, tasks per chunk, scratch bytes */
+/* split: the residue split that the whole-cube kernels would need at this grid
+ * (1: a product's cube fits a work-group's LDS; grids above 1 always take the
+ * streaming kernels), tasks per chunk, scratch bytes */
 int dgfs_bi_collision_plan_query(dgfs_bi_collision_plan_t plan, int* split, int* chunk,
                                  size_t* scratch_bytes);
+/* streaming: 1 where the plan's calls take the streaming kernels, 0 the
+ * whole-cube kernels; like_chunk: tasks per chunk of the calls whose opposite
+ * directions share a product (dgfs_bi_collide_like), 0 where none share */
+int dgfs_bi_collision_plan_form(dgfs_bi_collision_plan_t plan, int* streaming, int* like_chunk);
 /* Q_p[out] += prefac (gain - f_p loss) of the pair for every task: replaces
  * the per-node fs(cases[q], d_f, d_g, d_ux, e, r, m) loop of rhs()
  * (dgfs1D/bi/bi.py:329-337, scattering.py:261-321).  The task table is that

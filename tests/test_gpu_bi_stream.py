@@ -1,8 +1,8 @@
 """The mixture operator's streaming kernels (packed real transforms, Hermitian
 half of the products, paired directions) against the FP64 oracle and against
-each other, at the forms they accept: N = 20, 24, 32 with one and two lanes per
-plane row, rules with and without opposite directions, the like-species call,
-task chunks and several group and x-range splits.
+each other, at the forms they accept: N = 20, 24, 32, 48 with one and two lanes
+per plane row, rules with and without opposite directions, the like-species
+call, task chunks and several group and x-range splits.
 
 States carry 5 % noise, so that the Nyquist planes hold as much as the rest.
 Tolerances as tests/test_gpu_bivss.py: 1e-11 (FP64) and 3e-5 (FP32) of
@@ -24,15 +24,15 @@ def _rule(M, antipodal):
     return p / np.linalg.norm(p, axis=1)[:, None]
 
 
-def _call(cuda, N, M, antipodal, dtype, p, q, ntask_max, tasks=TASKS, masses=None, like=False,
-          Nrho=3, oracle=True):
+def _call(cuda, N, M, antipodal, dtype, p, q, ntask_max, tasks=TASKS, like=False, Nrho=3,
+          oracle=True):
     """Q of one call, its error against the oracle, and the plan's query."""
     import torch
     from dgfs1d_gpu_amd import _lib
     from dgfs1d_gpu_amd.collision import BiCollisionPlan
     vm = _mesh(N, 6, Nrho)
     sz, szpre = _rule(M, antipodal), load_design('womersley', 32)
-    m = masses or vm.masses
+    m = vm.masses
     u = _fields(vm, 2, 2, 11)
     plan = BiCollisionPlan(N, M, Nrho, vm.L, vm.qz, vm.qw, sz, vm.sw, szpre, m[p], m[q], 1.36,
                            0.8, 0.41, dtype, ntask_max, device=cuda)
@@ -57,13 +57,14 @@ def _call(cuda, N, M, antipodal, dtype, p, q, ntask_max, tasks=TASKS, masses=Non
 
 
 @pytest.mark.parametrize('N,dtype', [(20, 'F64'), (20, 'F32'), (24, 'F64'), (24, 'F32'),
-                                     (32, 'F64'), (32, 'F32')])
+                                     (32, 'F64'), (32, 'F32'), (48, 'F32')])
 @pytest.mark.parametrize('M,antipodal', [(6, True), (5, False), (1, False)])
 def test_rules(cuda, N, dtype, M, antipodal):
     from dgfs1d_gpu_amd import _lib
     # a task capacity whose product cubes exceed the streaming line at N = 20, 24
     got, err, info = _call(cuda, N, M, antipodal, getattr(_lib, dtype), 0, 1, 400 // M)
     print(N, dtype, M, antipodal, err, info, flush=True)
+    assert info['streaming'] and not info['like_chunk']       # unequal masses
     assert err < (1e-11 if dtype == 'F64' else 3e-5)
 
 
@@ -76,7 +77,7 @@ SAME = [(0, [(0, 1.0)], [(0, 1.0)]), (1, [(1, 0.5), (3, 0.25)], [(1, 0.5), (3, 0
         (1, [(2, -1.0)], [(2, -1.0)])]
 
 
-@pytest.mark.parametrize('N,dtype', [(20, 'F64'), (24, 'F32'), (32, 'F64')])
+@pytest.mark.parametrize('N,dtype', [(20, 'F64'), (24, 'F32'), (32, 'F64'), (48, 'F32')])
 @pytest.mark.parametrize('M,antipodal', [(6, True), (5, False)])
 @pytest.mark.parametrize('tasks', ['same', 'triplets'])
 def test_like_species(cuda, N, dtype, M, antipodal, tasks):
@@ -86,7 +87,8 @@ def test_like_species(cuda, N, dtype, M, antipodal, tasks):
     from dgfs1d_gpu_amd import _lib
     d = getattr(_lib, dtype)
     todo = SAME if tasks == 'same' else TRIPLETS
-    a, err, _ = _call(cuda, N, M, antipodal, d, 1, 1, 400 // M, todo, like=True)
+    a, err, info = _call(cuda, N, M, antipodal, d, 1, 1, 400 // M, todo, like=True)
+    assert info['streaming'] and (info['like_chunk'] > 0) == antipodal
     b, _, _ = _call(cuda, N, M, antipodal, d, 1, 1, 400 // M, todo, oracle=False)
     diff = np.abs(a - b).max() / np.abs(b).max()
     print(N, dtype, M, err, diff, flush=True)
@@ -97,15 +99,35 @@ def test_like_species(cuda, N, dtype, M, antipodal, tasks):
 def test_one_species_with_unsymmetric_tasks(cuda):
     """up is uq, but f and g do not exchange: the general form."""
     from dgfs1d_gpu_amd import _lib
-    a, err, _ = _call(cuda, 20, 6, True, _lib.F64, 0, 0, 70, TASKS, like=True)
+    a, err, info = _call(cuda, 20, 6, True, _lib.F64, 0, 0, 70, TASKS, like=True)
+    assert info['streaming'] and info['like_chunk']
     assert err < 1e-11
 
 
 def test_like_call_of_unequal_masses(cuda):
     """The like form needs equal masses: with others the call is the general one."""
+    import torch
     from dgfs1d_gpu_amd import _lib
-    a, err, _ = _call(cuda, 20, 6, True, _lib.F64, 0, 0, 70, SAME, masses=[1.0, 2.0], like=True)
-    assert err < 1e-11
+    from dgfs1d_gpu_amd.collision import BiCollisionPlan
+    N, M = 20, 6
+    vm = _mesh(N, M, 3)
+    sz, szpre, u = load_design('womersley', M), load_design('womersley', 32), _fields(vm, 2, 2, 11)[0]
+    d = torch.tensor(u, device=cuda)
+    for mp, mq in ((vm.masses[0], vm.masses[1]), (vm.masses[1], vm.masses[1])):
+        plan = BiCollisionPlan(N, M, 3, vm.L, vm.qz, vm.qw, sz, vm.sw, szpre, mp, mq, 1.36, 0.8,
+                               0.41, _lib.F64, 70, device=cuda)
+        info = plan.query()
+        assert info['streaming'] and (info['like_chunk'] > 0) == (mp == mq)
+        plan.set_tasks(2, 2, SAME)
+        Q = torch.zeros_like(d)
+        plan(d, d, Q)
+        plan.close()
+        pre = OB.BiPrecomp(N, vm.L, vm.qz, vm.qw, sz, vm.sw, szpre, mp, mq, 1.36, 0.8)
+        ref = np.zeros_like(u)
+        for out, ft, gt in SAME:
+            ref[out] += OB.q_pq(pre, sum(c * u[s] for s, c in ft), sum(c * u[s] for s, c in gt),
+                                0.41)
+        assert np.abs(Q.cpu().numpy() - ref).max() < 1e-11 * np.abs(ref).max()
 
 
 @pytest.mark.parametrize('N,dtype', [(20, 'F64'), (24, 'F32'), (16, 'F64')])
@@ -118,6 +140,7 @@ def test_engine_and_streaming_agree(cuda, N, dtype):
     b, eb, ib = _call(cuda, N, 6, True, d, 0, 1, 80)
     diff = np.abs(a - b).max() / np.abs(a).max()
     print(N, dtype, ea, eb, diff, ia, ib, flush=True)
+    assert not ia['streaming'] and ib['streaming'] == (N > 16)
     assert max(ea, eb) < (1e-11 if dtype == 'F64' else 3e-5)
     assert diff < (1e-13 if dtype == 'F64' else 3e-5)
 
@@ -266,11 +289,13 @@ def test_chunks(cuda, monkeypatch, like):
     def call(oracle):
         return _call(cuda, 32, 6, True, _lib.F64, 0, q, len(todo), todo, like=like, oracle=oracle)
     ref, err, info = call(True)
+    assert info['streaming'] and (info['like_chunk'] > 0) == like
     assert err < 1e-11
     seen = {info['chunk']}
     for mb in ('1', '22'):
         monkeypatch.setenv('DGFS_BI_SCRATCH_MB', mb)
         got, _, info = call(False)
         seen.add(info['chunk'])
+        assert info['like_chunk'] == (min(2 * info['chunk'], len(todo)) if like else 0)
         assert np.abs(got - ref).max() < 1e-13 * np.abs(ref).max()
     assert seen == {1, 2, len(todo)}, seen

@@ -88,8 +88,8 @@ def test_bi_collision_fp64(cuda, N, M, Nrho, Mpre, pq):
 @pytest.mark.parametrize('N,M,Nrho,Mpre', [(24, 6, 4, 32), (32, 6, 4, 32)])
 @pytest.mark.parametrize('pq', [(0, 1), (1, 1)])
 def test_bi_collision_fp64_slab_path(cuda, N, M, Nrho, Mpre, pq):
-    """Grids whose gain cube needs a residue split run the two-kernel slab
-    path (k_bi_yz, k_bi_xprod)."""
+    """FP64 grids whose product cube does not fit a work-group's LDS whole (its
+    split is above 1) take the streaming kernels at every plan size."""
     from dgfs1d_gpu_amd import _lib
     err, info = _run(cuda, N, M, Nrho, Mpre, _lib.F64, *pq)
     print('bi fp64 slab', N, pq, err, info, flush=True)
@@ -130,7 +130,7 @@ def test_bi_collision_chunked(cuda, monkeypatch):
 
 def test_bi_collision_fp32_n48(cuda):
     """N = 48 (the mixture grid of the reference's largest published runs),
-    FP32 on the slab path; FP64 at N = 48 is refused with an error."""
+    FP32 on the streaming kernels; FP64 at N = 48 is refused with an error."""
     from dgfs1d_gpu_amd import _lib
     err, info = _run(cuda, 48, 6, 2, 32, _lib.F32, 0, 1, tasks=TASKS[:2])
     print('bi fp32 n48', err, info, flush=True)

@@ -16,7 +16,7 @@
 // * f, g are real, so u1, u2 are real except for the Nyquist set (some index
 //   equal to N/2, which has no +N/2 partner), and one transform of
 //   X1 + i X2 carries both: w = IFFT3(X1 + i X2) = u1 + i u2.  With
-//   beta = Im u1, delta = Im u2 (from the Nyquist planes alone, k_bi_nyq),
+//   beta = Im u1, delta = Im u2 (from the Nyquist planes alone, BiNyq),
 //   Re u1 = Re w + delta, Re u2 = Im w - beta.  The spectrum of
 //   beta + i delta is K = kap1 F + i kap2 G, kap = (e - e~)/(2i), e the
 //   phase and e~ the phase with the conjugate factor on every Nyquist axis.
@@ -35,10 +35,12 @@
 //
 // Measured (FP64 N = 32, M = 12, N_rho = 8, 216 tasks per pair, four pairs; one
 // call): 101.9 ms as complex transforms of both sides and the product, 29.9 ms
-// here.  Shares: k_bi_plane 44 % (vector units 56 % busy, half the LDS cycles
-// are conflicts of the exchanges; three waves per SIMD spill: 28 -> 33 ms),
-// k_bi_x 26 % and k_bi_sum 23 % (near the HBM rate of the products they write
-// and read), k_bi_pen 2 %.  N = 20: 12.9 -> 7.8 ms; FP32 N = 48: 157 -> 38 ms.
+// here.  Shares: k_bi_plane 44 %, k_bi_x 26 % and k_bi_sum 23 % (near the HBM
+// rate of the products they write and read), k_bi_pen 2 %.  N = 20: 12.9 -> 7.8
+// ms; FP32 N = 48: 157 -> 38 ms.  k_bi_plane by counters, N = 32, 20, 48: vector
+// units busy 52, 53, 62 %, LDS 36, 22, 22 % of the busy cycles, of its cycles
+// 50, 16, 37 % bank conflicts of the exchanges; three waves per SIMD spill (N =
+// 32: 28 -> 33 ms).
 //
 // Layouts: pencil p(l2, l3) = (l3 / 2) 2N + 2 l2 + (l3 & 1), the order in
 // which k_bi_plane's lanes hold a plane; F[which][l1][p]; Y[d][x][p], whose
@@ -46,8 +48,9 @@
 // with q the regular pencils k3 <= N/2 (same formula), then the lines
 // (k2 = N/2, k3 = 0..N/2) and (k2, k3 = N/2).  In place a product takes 0.57
 // instead of 0.9 MB (FP64 N = 32), so a chunk of the scratch budget holds 1.6
-// times the tasks.  spec[d][s][q]: the k1 = N/2 plane of x-range s.  Every length-N transform is shared
-// by a lane pair (pair_dft_*): half the registers per lane.
+// times the tasks.  spec[d][s][q]: the k1 = N/2 plane of x-range s.  Every
+// length-N transform is shared by a lane pair (pair_dft_*), but for k_bi_plane's
+// at N = 20: half the registers per lane.
 #pragma once
 #include "collision_kernels.h"
 
@@ -321,8 +324,7 @@ template <typename T, int N>
 struct BiPlane {
     static constexpr int LN = bi_lanes(N), PN = N / LN, H = N / 2, PT = LN * N;
     static constexpr int PW = LN == 1 ? 64 / N
-                                      : (PT % 64 == 0 ? 1 : PT % 32 == 0 ? 2 : PT % 16 == 0 ? 4
-                                                                         : PT % 8 == 0 ? 8 : 16);
+                                      : (PT % 64 == 0 ? 1 : PT % 32 == 0 ? 2 : 4);
     static constexpr int WG = LN == 1 ? 64 : PW * PT;
     static_assert(WG % 64 == 0 && PW >= 1, "whole waves");
     static constexpr int PI = N + 1, ELEMS = N * PI;

@@ -397,16 +397,18 @@ template <typename T, int N>
 int bi_stream_tables(BiPlan* pl, const int* ylist, const double* fac, const double* wx,
                      const double* szpre, const double* Bt, const double* wc, const double* Bsum,
                      double mqf) {
-    if constexpr (!bi_streams(N)) return 1;
-    using Gm = BiGeo<N>;
-    hipLaunchKernelGGL((k_bi_chtab<T, N>), dim3((N * Gm::NPH + 31) / 32), dim3(256), 0, 0,
-                       pl->Nrho, pl->Mpre, fac, wc, szpre, Bsum, (cplx<T>*)pl->ctab);
-    const int us = pl->antipodal ? 2 : 1, NU = pl->Nrho * pl->M / us;
-    const long per = long(N) * Gm::NPT + Gm::NPH;
-    hipLaunchKernelGGL((k_bi_wtab<T, N>), dim3((NU * per + 255) / 256), dim3(256), 0, 0, pl->M, NU,
-                       us, pl->Mpre, ylist, fac, wx, szpre, Bt, mqf, (cplx<T>*)pl->wtab,
-                       (cplx<T>*)pl->wspec);
-    return hipGetLastError() == hipSuccess ? 0 : 1;
+    if constexpr (bi_streams(N)) {
+        using Gm = BiGeo<N>;
+        hipLaunchKernelGGL((k_bi_chtab<T, N>), dim3((N * Gm::NPH + 31) / 32), dim3(256), 0, 0,
+                           pl->Nrho, pl->Mpre, fac, wc, szpre, Bsum, (cplx<T>*)pl->ctab);
+        const int us = pl->antipodal ? 2 : 1, NU = pl->Nrho * pl->M / us;
+        const long per = long(N) * Gm::NPT + Gm::NPH;
+        hipLaunchKernelGGL((k_bi_wtab<T, N>), dim3((NU * per + 255) / 256), dim3(256), 0, 0,
+                           pl->M, NU, us, pl->Mpre, ylist, fac, wx, szpre, Bt, mqf,
+                           (cplx<T>*)pl->wtab, (cplx<T>*)pl->wspec);
+        return hipGetLastError() == hipSuccess ? 0 : 1;
+    }
+    return 1;
 }
 
 #define DGFS_BI_SIG(T, N)                                                                  \

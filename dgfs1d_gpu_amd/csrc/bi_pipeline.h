@@ -67,7 +67,7 @@ struct BiGeo {
     static_assert(N < 20 || NPT <= NN, "a plane's results fit its place in Y");
     static DGFS_HD int pen(int l2, int l3) { return (l3 / 2) * 2 * N + 2 * l2 + (l3 & 1); }
 };
-constexpr int kBiXSMax = 12;                        // most x-ranges of a product
+constexpr int kBiXSMax = 16;                        // most x-ranges of a product
 
 // F[t][which][k1][p] = FFT_x(Iw)/n, one thread per (t, which, p), and
 // norm[t][which][0][blk] = the work-group's sum of |F|^2, 0 only where F is zero.

@@ -230,6 +230,11 @@ struct BiPlan {
 // weights).  Against the first split of at least 2048 waves, same chunks: N = 20
 // FP64 8.11 -> 7.83 ms, N = 48 FP32 41.9 -> 38.0, N = 32 FP64 29.7 both, the
 // 6-task N = 24 set 536/538 us (at 4096 waves it took 591).
+// A group also costs k_bi_pen a step of its serial sum (0.3 weights): one task
+// of 96 directions, N = 24 FP64, 374 us without that term, 356 with it.  More
+// than 12 ranges only where four work-groups per CU or fewer come of it, because
+// k_bi_sum adds their k1 = N/2 planes up: N = 32 FP32, one task of 30 directions
+// 270 -> 252 us, but of 216 directions 465 -> 504.
 constexpr int kBiCU = 256;
 inline double bi_share(long blocks, int wg, double length) {
     const long per = (blocks + kBiCU - 1) / kBiCU;
@@ -241,8 +246,9 @@ inline int bi_xranges(int nt, int ND) {
     int XS = 1;
     double least = 0.0;
     for (int d = 1; d <= kBiXSMax; ++d) {
-        if (N % d) continue;
-        const double c = bi_share((long(nt) * ND * d + Pl::PW - 1) / Pl::PW, Pl::WG, N / d + 0.5);
+        const long blocks = (long(nt) * ND * d + Pl::PW - 1) / Pl::PW;
+        if (N % d || (d > 12 && blocks > 4 * kBiCU)) continue;
+        const double c = bi_share(blocks, Pl::WG, N / d + 0.5);
         if (d == 1 || c < least) XS = d, least = c;
     }
     return XS;
@@ -250,12 +256,14 @@ inline int bi_xranges(int nt, int ND) {
 template <int N>
 inline int bi_sum_groups(int nt, int NU) {
     constexpr int QB = (BiGeo<N>::NPT + kBiSumWG / 2 - 1) / (kBiSumWG / 2);
+    constexpr int QF = (BiGeo<N>::NPH + 31) / 32;
     int XG = 1;
     double least = 0.0;
     for (int per = NU; per >= 1; --per) {
         const int g = (NU + per - 1) / per;
         if (g > 64) break;
-        const double c = bi_share(long(nt) * QB * g, kBiSumWG, per + 2.0);
+        const double c = bi_share(long(nt) * QB * g, kBiSumWG, per + 2.0) +
+                         bi_share(long(nt) * QF, kBiPenWG, 0.3 * g);
         if (per == NU || c < least) XG = g, least = c;
     }
     return XG;
